@@ -36,21 +36,20 @@ __global__ void k_batch_reset(uint32_t* counters) {
     if (threadIdx.x < kClasses * kQueues) counters[threadIdx.x] = 0;
 }
 
-// PIPE: the DDA loads the next steps' macro words while it gathers the
-// current ones (more registers; used by the DDA class kernel, whose register
-// budget is its own, not by the all-class kernel).  For a DDA view,
-// lds_mask says that `lds` holds this wave's copy of the view's macro
-// bitmask: the loop then reads the mask from LDS, as the plain kernel does.
-template <int TRAV, bool PIPE = (TRAV == XD_DDA)>
+// For a DDA view, lds_mask says that `lds` holds this wave's copy of the view's
+// macro bitmask: the loop then reads the mask from LDS, as the plain kernel
+// does.  RUN: see dda_trace; the DDA class kernel has a register budget of its
+// own, the all-class kernel takes the shorter batch.
+template <int TRAV, uint32_t RUN = kDdaRun>
 __device__ __forceinline__ void shade_tile(const BatchView& V, uint32_t tile, uint32_t lane, uint32_t* lds,
                                            bool lds_mask = false);
 
 // Any traversal: the kernel for all classes at once dispatches on the view.
 template <>
-__device__ __forceinline__ void shade_tile<kClasses, false>(const BatchView& V, uint32_t tile, uint32_t lane,
+__device__ __forceinline__ void shade_tile<kClasses, kDdaRun>(const BatchView& V, uint32_t tile, uint32_t lane,
                                                             uint32_t* lds, bool lds_mask) {
     switch (V.traversal) {
-    case XD_DDA: shade_tile<XD_DDA, false>(V, tile, lane, lds, lds_mask); break;
+    case XD_DDA: shade_tile<XD_DDA, kDdaRunAll>(V, tile, lane, lds, lds_mask); break;
     case XD_SVO_NAIVE: shade_tile<XD_SVO_NAIVE>(V, tile, lane, lds); break;
     case XD_ESVO: shade_tile<XD_ESVO>(V, tile, lane, lds); break;
     case XD_SVO_DF: shade_tile<XD_SVO_DF>(V, tile, lane, lds); break;
@@ -58,7 +57,7 @@ __device__ __forceinline__ void shade_tile<kClasses, false>(const BatchView& V, 
     }
 }
 
-template <int TRAV, bool PIPE>
+template <int TRAV, uint32_t RUN>
 __device__ __forceinline__ void shade_tile(const BatchView& V, uint32_t tile, uint32_t lane, uint32_t* lds,
                                            bool lds_mask) {
     const uint32_t sh = V.tw_shift;
@@ -76,11 +75,11 @@ __device__ __forceinline__ void shade_tile(const BatchView& V, uint32_t tile, ui
         const f3 ro = muls(p.cam.translation, side);
         coeff = emission_coeff(p.view, rd) / side;
         if (lds_mask)
-            c = p.wide ? dda_trace<false, true, false>(p, lds, ro, rd, words)
-                       : dda_trace<false, false, false>(p, lds, ro, rd, words);
+            c = p.wide ? dda_trace<false, true, RUN>(p, lds, ro, rd, words)
+                       : dda_trace<false, false, RUN>(p, lds, ro, rd, words);
         else
-            c = p.wide ? dda_trace<false, true, PIPE>(p, p.macro, ro, rd, words)
-                       : dda_trace<false, false, PIPE>(p, p.macro, ro, rd, words);
+            c = p.wide ? dda_trace<false, true, RUN>(p, p.macro, ro, rd, words)
+                       : dda_trace<false, false, RUN>(p, p.macro, ro, rd, words);
     } else {
         c = p.cw ? svo_pixel<TRAV, false, true, false>(p, rd, lds, nullptr, words)
                  : svo_pixel<TRAV, false, false, false>(p, rd, lds, nullptr, words);

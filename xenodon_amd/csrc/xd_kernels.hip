@@ -32,7 +32,7 @@ __global__ __launch_bounds__(256) void k_dda(RenderParams p) {
         float side = max_elem(mk((float)p.dims[0], (float)p.dims[1], (float)p.dims[2]));
         f3 ro = muls(p.cam.translation, side);
         float ec = emission_coeff(p.view, rd) / side;
-        f3 total = dda_trace<COUNT, WIDE>(p, lds_macro, ro, rd, words);
+        f3 total = dda_trace<COUNT, WIDE, kDdaRun>(p, lds_macro, ro, rd, words);
         if (!COUNT) p.out[(uint64_t)iy * p.out_pitch + ix] = pack_rgba(muls(total, ec));
     }
     if (COUNT) add_words(p.words, words);
@@ -148,9 +148,10 @@ __global__ __launch_bounds__(256) void k_macro_mask(const uint8_t* __restrict__ 
         if (cell >= mnx * mny * mnz) break;
         const uint32_t cx = cell % mnx, cy = (cell / mnx) % mny, cz = cell / (mnx * mny);
         uint32_t any = 0;
-        for (uint32_t bz = cz << bshift; bz < min(nbz, (cz + 1) << bshift) && !any; ++bz)
-            for (uint32_t by = cy << bshift; by < min(nby, (cy + 1) << bshift) && !any; ++by)
-                for (uint32_t bx = cx << bshift; bx < min(nbx, (cx + 1) << bshift); ++bx)
+        const uint32_t x0 = cx << bshift, y0 = cy << bshift, z0 = cz << bshift, side = (1u << bshift) + 2u;
+        for (uint32_t bz = z0 > 1 ? z0 - 2 : 0; bz < min(nbz, z0 + side) && !any; ++bz)
+            for (uint32_t by = y0 > 1 ? y0 - 2 : 0; by < min(nby, y0 + side) && !any; ++by)
+                for (uint32_t bx = x0 > 1 ? x0 - 2 : 0; bx < min(nbx, x0 + side); ++bx)
                     if (occ[((uint64_t)bz * nby + by) * nbx + bx]) {
                         any = 1;
                         break;
