@@ -1,0 +1,51 @@
+"""The batched forms' tile queues: launches from one wave tile up to more tiles
+than resident waves, growing and shrinking on one batch object (whose captured
+launch is reused), give the plain render's frames, bit for bit."""
+import numpy as np
+import pytest
+
+from tests import helpers as H
+from xenodon_amd import abi
+
+pytestmark = pytest.mark.gpu
+
+TRAVERSALS = [abi.DDA, abi.SVO_NAIVE, abi.ESVO, abi.SVO_DF, abi.SVO_ROPE]
+# (views, width, height): 1 tile; one block; a few blocks; ~13000 tiles; small again
+SHAPES = [(1, 1, 1), (4, 8, 8), (5, 37, 29), (40, 161, 127), (2, 9, 8), (15, 64, 65)]
+
+
+@pytest.fixture(scope="module")
+def env():
+    if abi.device_count() < 1:
+        pytest.fail("no HIP device visible: GPU tests need an MI355X")
+    ctx = abi.Context(0)
+    grid = H.blocky_grid(32, 4, seed=5)
+    nodes, st = abi.build_octree(grid, tree=abi.TREE_ROPE)
+    yield ctx, (ctx.grid_volume(grid), [32] * 3), (ctx.svo_volume(nodes, st["side"]), [st["side"]] * 3)
+    ctx.close()
+
+
+@pytest.mark.parametrize("travs", [[t] for t in TRAVERSALS] + [TRAVERSALS])
+@pytest.mark.parametrize("class_kernels,waves,grab", [(0, 8, 1), (1, 0, 4)])
+def test_queue_sizes_match_plain_renders(env, travs, class_kernels, waves, grab):
+    ctx, grid, svo = env
+    b = ctx.batch()
+    b.set_tuning([8] * 5, tiles_per_grab=grab, waves_per_simd=waves, class_kernels=class_kernels)
+    for n, W, Hh in SHAPES:
+        views = []
+        for k, (f, up, eye) in enumerate(H.orbit_cameras(n, 1.6, seed=n)):
+            t = travs[k % len(travs)]
+            vol, md = grid if t == abi.DDA else svo
+            views.append((vol, t, abi.make_camera(f, up, eye), abi.make_uniforms(W, Hh, md, emission=1.5),
+                          ctx.frame(W, Hh)))
+        refs = [ctx.render_image(*v[:4])[0] for v in views]
+        b.set_views(views)
+        for _ in range(2):
+            b.render()
+            for v, ref in zip(views, refs):
+                assert np.array_equal(v[4].download(), ref), (n, W, Hh)
+        abi.render_static(ctx, views, {"tile_w": [8] * 5, "class_kernels": class_kernels})
+        for v, ref in zip(views, refs):
+            assert np.array_equal(v[4].download(), ref), (n, W, Hh, "static")
+            v[4].free()
+    b.free()

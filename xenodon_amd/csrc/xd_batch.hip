@@ -33,7 +33,7 @@
 namespace xd {
 
 __global__ void k_batch_reset(uint32_t* counters) {
-    if (threadIdx.x < kClasses * kQueues) counters[threadIdx.x] = 0;
+    if (threadIdx.x < kClasses * kQueues) counters[threadIdx.x * kCounterStride] = 0;
 }
 
 // For a DDA view, lds_mask says that `lds` holds this wave's copy of the view's
@@ -91,7 +91,12 @@ __device__ __forceinline__ void shade_tile(const BatchView& V, uint32_t tile, ui
 // The tiles of one traversal class: kQueues ranges (one per XCD) of
 // qbeg/counters.  A wave takes tiles from its own XCD's range with one atomic
 // per grab and moves on to the other ranges when that one is drained; every
-// wave leaves once all ranges are drained.  grabs packs the tiles per grab of
+// wave leaves once all ranges are drained.  To choose a range it reads every
+// range's counter with one load, a lane each, and takes the first in its order
+// that is not drained: an atomic on each drained range in turn, 40 of them by
+// each of 8192 waves at 5 ns on a shared cache line, had cost 1.7 ms a launch
+// (0.7 ms in a class kernel's 8 ranges), however little work there was.
+// grabs packs the tiles per grab of
 // each class, 6 bits each (class c at bit 6c).
 template <int TRAV>
 __device__ __forceinline__ void class_body(const BatchView* __restrict__ views, const uint32_t* __restrict__ tiles,
@@ -108,17 +113,27 @@ __device__ __forceinline__ void class_body(const BatchView* __restrict__ views, 
     // in the all-class kernel (whose esvo and svo-df tiles overwrite it).  A
     // mask larger than the region is read from device memory.
     const uint32_t* staged = nullptr;
-    for (uint32_t qi = 0; qi < kRanges; ++qi) {
-        // this XCD's range first (of every class, for the all-class kernel),
-        // then the next XCD's
-        const uint32_t qq = TRAV == (int)kClasses
-                                ? ((qi + first) % kClasses) * kQueues + (home + qi / kClasses) % kQueues
-                                : (home + qi) % kQueues;
+    uint64_t drained = 0;  // places in this wave's order whose range it has seen the end of
+    for (;;) {
+        // lane p: the p-th range in this wave's order, this XCD's first (of
+        // every class, for the all-class kernel), then the next XCD's
+        const uint32_t range = TRAV == (int)kClasses
+                                   ? ((lane + first) % kClasses) * kQueues + (home + lane / kClasses) % kQueues
+                                   : (home + lane) % kQueues;
+        bool open = false;
+        if (lane < kRanges)
+            open = __hip_atomic_load(&counters[range * kCounterStride], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) <
+                   qbeg[range + 1] - qbeg[range];
+        const uint64_t left = __builtin_amdgcn_ballot_w64(open) & ~drained;
+        if (left == 0) break;
+        const uint32_t place = (uint32_t)__builtin_ctzll(left);
+        drained |= 1ull << place;  // it is, when the loop below ends
+        const uint32_t qq = __builtin_amdgcn_readlane(range, place);
         const uint32_t beg = qbeg[qq], end = qbeg[qq + 1];
         const uint32_t per_grab = (grabs >> (6u * (TRAV == (int)kClasses ? qq / kQueues : (uint32_t)TRAV))) & 63u;
         for (;;) {
             uint32_t t = 0;
-            if (lane == 0) t = atomicAdd(&counters[qq], per_grab);
+            if (lane == 0) t = atomicAdd(&counters[qq * kCounterStride], per_grab);
             // wave-uniform from here on: the view's parameters are read with
             // scalar loads into SGPRs instead of occupying VGPRs
             t = __builtin_amdgcn_readfirstlane(t);
@@ -220,6 +235,11 @@ size_t batch_lds_bytes(int traversal, uint32_t slots) {
     return slots ? (size_t)2 * slots * kBlockThreads * sizeof(uint32_t) : 0;
 }
 
+uint32_t grid_for_tiles(uint32_t resident, uint64_t tiles) {
+    const uint64_t blocks = (tiles + kBlockThreads / kWaveLanes - 1) / (kBlockThreads / kWaveLanes);
+    return (uint32_t)std::min<uint64_t>(resident, (blocks + kQueues - 1) / kQueues * kQueues);
+}
+
 int batch_grid(int device, int traversal, uint32_t slots, bool w8, uint32_t* grid) {
     hipError_t e;
     int cus = 0, per_cu = 0;
@@ -240,7 +260,7 @@ hipError_t launch_batch(const BatchView* views, const uint32_t* tiles, const uin
         if (!cls.grid[c]) continue;  // no tiles for this kernel
         const uint32_t base = c < (int)kClasses ? c * kQueues : 0;
         hipLaunchKernelGGL(kKernels[w8][c], dim3(cls.grid[c]), dim3(256), batch_lds_bytes(c, cls.slots[c]), s, views,
-                           tiles, qbeg + base, counters + base, grabs, mix ? 1u : 0u);
+                           tiles, qbeg + base, counters + base * kCounterStride, grabs, mix ? 1u : 0u);
     }
     return hipGetLastError();
 }
@@ -265,6 +285,7 @@ struct xd_batch {
     hipGraphExec_t exec = nullptr;
     BatchClasses graph_cls{};  // per-class grids and LDS stack strides the graph was captured with
     uint32_t graph_grab = 0, graph_w8 = 0, graph_mix = 0;
+    uint32_t resident[kClasses + 1] = {};  // resident blocks of each captured kernel
     bool keep_mixed = false;  // autotuner: one traversal's views on the all-traversal kernel
 };
 
@@ -432,8 +453,8 @@ int build_tables(const xd_view* views, uint32_t n, const xd_batch_tuning& tuning
         }
     // A batch of one traversal runs that traversal's own kernel whatever the
     // tuning says: with one class there is nothing to mix, and the class
-    // kernel has that traversal's register budget (and, for DDA, the loop
-    // that loads the next steps' macro words during the current gathers).
+    // kernel has that traversal's register budget (and, for DDA, the longer
+    // batches of steps).
     uint32_t present = 0;
     for (uint32_t c = 0; c < kClasses; ++c) present += cls.grid[c] ? 1u : 0u;
     const bool per_class = tuning.class_kernels || (present == 1 && !keep_mixed);
@@ -462,6 +483,8 @@ int build_tables(const xd_view* views, uint32_t n, const xd_batch_tuning& tuning
     T.tiles.clear();
     T.tiles.reserve(total);
     for (auto& v : q) T.tiles.insert(T.tiles.end(), v.begin(), v.end());
+    for (uint32_t c = 0; c < kClasses; ++c) cls.tiles[c] = T.qbeg[(c + 1) * kQueues] - T.qbeg[c * kQueues];
+    cls.tiles[kClasses] = (uint32_t)total;
     T.cls = cls;
     return XD_OK;
 }
@@ -493,8 +516,13 @@ int capture(xd_batch* b, const BatchClasses& need) {
     BatchClasses cls = need;
     for (int c = 0; c <= (int)kClasses; ++c) {
         if (!need.grid[c]) continue;
-        int rc = batch_grid(b->ctx->device, c, need.slots[c], w8, &cls.grid[c]);
+        int rc = batch_grid(b->ctx->device, c, need.slots[c], w8, &b->resident[c]);
         if (rc) return rc;
+        // rounded up to a power of two blocks, so that view sets of growing
+        // size capture a few times at most
+        uint32_t blocks = kQueues;
+        while (blocks < grid_for_tiles(b->resident[c], need.tiles[c])) blocks *= 2;
+        cls.grid[c] = std::min(blocks, b->resident[c]);
     }
     hipStream_t s = b->ctx->stream;
     const uint32_t grab = pack_grabs(b->tuning.tiles_per_grab, b->tuning.rays_per_lane);
@@ -521,7 +549,9 @@ int prepare(xd_batch* b) {
     bool stale = !b->exec || grab != b->graph_grab || b->graph_w8 != (uint32_t)(b->tuning.waves_per_simd == 8) ||
                  b->graph_mix != b->tuning.mix_classes;
     for (int c = 0; c <= (int)kClasses; ++c)
-        stale |= (need.grid[c] && !b->graph_cls.grid[c]) || need.slots[c] > b->graph_cls.slots[c];
+        stale |= (need.grid[c] && (!b->graph_cls.grid[c] ||
+                                   b->graph_cls.grid[c] < grid_for_tiles(b->resident[c], need.tiles[c]))) ||
+                 need.slots[c] > b->graph_cls.slots[c];
     return stale ? capture(b, need) : XD_OK;
 }
 
@@ -604,7 +634,7 @@ int xd_batch_create(xd_context* ctx, xd_batch** out) {
     b->ctx = ctx;
     b->tuning = default_tuning();
     if ((e = hipMalloc(&b->d_qbeg, sizeof(uint32_t) * (kClasses * kQueues + 1))) != hipSuccess ||
-        (e = hipMalloc(&b->d_counters, sizeof(uint32_t) * kClasses * kQueues)) != hipSuccess) {
+        (e = hipMalloc(&b->d_counters, kCounterBytes)) != hipSuccess) {
         xd_batch_free(b);
         return fail_hip(e, "batch allocation");
     }
@@ -758,7 +788,7 @@ constexpr uint32_t kStaticTiles = 1u << 21;  // 2M wave tiles: 134M rays at 64 p
 constexpr size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 constexpr size_t kScratchQbeg = align256(sizeof(BatchView) * kStaticViews);
 constexpr size_t kScratchCounters = kScratchQbeg + align256(sizeof(uint32_t) * (kClasses * kQueues + 1));
-constexpr size_t kScratchTiles = kScratchCounters + align256(sizeof(uint32_t) * kClasses * kQueues);
+constexpr size_t kScratchTiles = kScratchCounters + align256(kCounterBytes);
 constexpr size_t kScratchBytes = kScratchTiles + sizeof(uint32_t) * kStaticTiles;
 static_assert(alignof(BatchView) <= 256, "view table alignment");
 
@@ -818,7 +848,10 @@ int xd_batch_render_static(xd_context* ctx, const xd_view* views, uint32_t count
     const bool w8 = tun.waves_per_simd == 8;
     BatchClasses cls = T.cls;
     for (int c = 0; c <= (int)kClasses; ++c)
-        if (cls.grid[c] && (rc = batch_grid(ctx->device, c, cls.slots[c], w8, &cls.grid[c]))) return rc;
+        if (cls.grid[c]) {
+            if ((rc = batch_grid(ctx->device, c, cls.slots[c], w8, &cls.grid[c]))) return rc;
+            cls.grid[c] = grid_for_tiles(cls.grid[c], cls.tiles[c]);
+        }
     BatchView* d_views = reinterpret_cast<BatchView*>(base);
     uint32_t* d_qbeg = reinterpret_cast<uint32_t*>(base + kScratchQbeg);
     uint32_t* d_counters = reinterpret_cast<uint32_t*>(base + kScratchCounters);

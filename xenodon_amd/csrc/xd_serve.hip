@@ -311,7 +311,7 @@ bool launch_step(xd_server* s, Step& S, std::string* err) {
     for (uint32_t c = 0; c <= kClasses; ++c) {
         const bool present = per_class ? (c < kClasses && count[c]) : c == kClasses;
         if (!present) continue;
-        cls.grid[c] = grid_for(s, (int)c, cls.slots[c]);
+        cls.grid[c] = grid_for_tiles(grid_for(s, (int)c, cls.slots[c]), c == kClasses ? n : count[c]);
         if (!cls.grid[c]) {
             *err = "served step: occupancy query failed";
             return false;
@@ -558,7 +558,7 @@ int xd_server_create(xd_context* ctx, const xd_server_config* cfg, xd_server** o
     s->views_off = 0;
     s->qbeg_off = (sizeof(BatchView) * c.max_active + 255) / 256 * 256;
     s->counters_off = s->qbeg_off + 256;  // qbeg: kClasses * kQueues + 1 entries
-    s->tiles_off = s->counters_off + 256;
+    s->tiles_off = s->counters_off + kCounterBytes;
     s->table_bytes = s->tiles_off + (size_t)c.tiles_per_launch * sizeof(uint32_t);
     s->read_streams.assign(c.readback_threads, nullptr);
     e = hipMalloc(&s->arena_dev, c.frame_arena_bytes);
