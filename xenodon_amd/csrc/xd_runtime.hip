@@ -443,9 +443,6 @@ int xd_volume_from_svo(xd_context* ctx, const void* nodes, uint64_t node_count, 
     if (node_count == 0) return fail(XD_ERR_FORMAT, "octree has no nodes");
     if (node_count > 0xFFFFFFFFull) return fail(XD_ERR_FORMAT, "octree has more than 2^32 nodes");
     const uint32_t* w = static_cast<const uint32_t*>(nodes);
-    uint32_t max_depth = 0, is_rope = 0;
-    int rc = analyse_octree(w, node_count, &max_depth, &is_rope);
-    if (rc) return rc;
     hipError_t e = hipSetDevice(ctx->device);
     if (e != hipSuccess) return fail_hip(e, "hipSetDevice");
     auto* v = new xd_volume();
@@ -454,11 +451,23 @@ int xd_volume_from_svo(xd_context* ctx, const void* nodes, uint64_t node_count, 
     v->side = side;
     v->dims[0] = v->dims[1] = v->dims[2] = side;
     v->node_count = node_count;
-    v->max_depth = max_depth;
-    v->is_rope = is_rope;
+    const bool tagged = node_count <= kMaxTaggedNodes && ctx->octree_layout != 1;
+    const bool wide = node_count > kMaxNarrowTagNodes || ctx->octree_layout == 2;
+    if (tagged && derive_layout_on_device(v, w, node_count, wide)) {
+        v->bytes = svo_footprint(node_count, false);
+        ctx->volumes.insert(v);
+        clear_error();
+        *out = v;
+        return XD_OK;
+    }
+    int rc = analyse_octree(w, node_count, &v->max_depth, &v->is_rope);
+    if (rc) {
+        delete v;
+        return rc;
+    }
     const uint64_t bytes = node_count * kNodeWords * sizeof(uint32_t);
     v->bytes = bytes;
-    if (node_count <= kMaxTaggedNodes && ctx->octree_layout != 1) {
+    if (tagged) {
         // tagged, sibling-grouped layout, derived on the host
         // every word is written by the derivation: no zero-fill of tens of GB
         std::unique_ptr<uint32_t[]> cw_buf(new (std::nothrow) uint32_t[node_count * 8]);
@@ -469,7 +478,6 @@ int xd_volume_from_svo(xd_context* ctx, const void* nodes, uint64_t node_count, 
         }
         uint32_t* const cw = cw_buf.get();
         uint32_t* const meta = meta_buf.get();
-        const bool wide = node_count > kMaxNarrowTagNodes || ctx->octree_layout == 2;
         // large trees (the converter's, not DAGs) are numbered and checked in parallel
         const bool tree = node_count >= (1ull << 22) && octree_is_tree(w, node_count);
         build_tagged_layout(w, node_count, cw, meta, v->top, wide, tree, &v->empty_start, &v->leaf_base);
@@ -501,19 +509,18 @@ int xd_volume_from_svo(xd_context* ctx, const void* nodes, uint64_t node_count, 
         meta_buf.reset();
         if ((e = hipMalloc(&v->d_cw, node_count * 8 * sizeof(uint32_t))) != hipSuccess ||
             (e = hipMalloc(&v->d_meta, node_count * 2 * sizeof(uint32_t))) != hipSuccess ||
-            (e = hipMemcpy(v->d_cw, planes.get(), cw_words * sizeof(uint32_t), hipMemcpyHostToDevice)) !=
-                hipSuccess ||
-            (e = hipMemcpy(v->d_meta, meta_planes.get(), node_count * 2 * sizeof(uint32_t), hipMemcpyHostToDevice)) !=
-                hipSuccess) {
+            (e = hipMemcpyAsync(v->d_cw, planes.get(), cw_words * sizeof(uint32_t), hipMemcpyHostToDevice,
+                                ctx->stream)) != hipSuccess ||
+            (e = hipMemcpyAsync(v->d_meta, meta_planes.get(), node_count * 2 * sizeof(uint32_t), hipMemcpyHostToDevice,
+                                ctx->stream)) != hipSuccess) {
             xd_volume_free(v);
             return fail_hip(e, "octree upload");
         }
         const uint32_t root_ld = w[9], root_col = w[8];
         v->root_tag = (root_ld & kLeafMask) ? (kTagLeaf | ((root_col & 0xFFFFFFu) ? 0u : v->empty_tag)) : 0u;
-        std::vector<uint2> table(kTableCells);
-        build_start_table(planes.get(), v->root_tag, v->index_mask, table.data());  // internal nodes' words as in cw
         if ((e = hipMalloc(&v->d_table, kTableBytes)) != hipSuccess ||
-            (e = hipMemcpy(v->d_table, table.data(), kTableBytes, hipMemcpyHostToDevice)) != hipSuccess) {
+            (e = launch_start_table(v->d_cw, v->root_tag, v->index_mask, nullptr, v->d_table, ctx->stream)) != hipSuccess ||
+            (e = hipStreamSynchronize(ctx->stream)) != hipSuccess) {
             xd_volume_free(v);
             return fail_hip(e, "octree upload");
         }

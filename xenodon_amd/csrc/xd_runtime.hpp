@@ -110,6 +110,15 @@ bool octree_depths_exact(const uint32_t* w, uint64_t n, bool tree);
 // child words for at most L levels, so any tree, cyclic ones included, gives
 // a table.
 void build_start_table(const uint32_t* child_w, uint32_t root_tag, uint32_t index_mask, uint2* table);
+// The same table built on the device, from the device form of child_w.  stop:
+// null, or a device word that, if set, keeps the table unwritten.
+hipError_t launch_start_table(const uint32_t* cw, uint32_t root_tag, uint32_t index_mask, const uint32_t* stop,
+                              uint2* table, hipStream_t s);
+// Derives v's tagged layout and start table on the device from n .svo nodes in
+// host memory, and sets everything of v that depends on them.  False if the
+// tree or the device memory does not allow it (see xd_octree.hip); v is as it
+// was then, and the host derivation decides.
+bool derive_layout_on_device(xd_volume* v, const uint32_t* w, uint64_t n, bool wide);
 // When the tree has fewer than 2^25 nodes and every depth field is below 32,
 // ORs into every child word of every leaf (its ropes) the depth field of the
 // node it points to, shifted by kRopeDepthShift, and returns true; else
