@@ -112,8 +112,8 @@ hipError_t launch_macro_mask(const uint8_t* occ, const uint32_t nb[3], uint32_t 
                              uint32_t* macro, uint32_t words, hipStream_t s);
 
 // Grid upload: rewrite `layers` z-layers (X*Y texels each, x fastest) held in
-// `staging` into bricks of brick-layer `bz`, and set the occupancy bytes.
-hipError_t launch_brick_layer(const uint32_t* staging, uint32_t layers, uint32_t bz, uint32_t* bricks, uint8_t* occ,
-                              const uint32_t dims[3], const uint32_t nb[3], hipStream_t s);
+// `staging` into bricks from brick-layer `bz` on, and set the occupancy bytes.
+hipError_t launch_bricks(const uint32_t* staging, uint32_t layers, uint32_t bz, uint32_t* bricks, uint8_t* occ,
+                         const uint32_t dims[3], const uint32_t nb[3], hipStream_t s);
 
 }  // namespace xd

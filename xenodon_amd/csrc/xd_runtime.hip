@@ -146,6 +146,9 @@ uint32_t macro_geometry(const uint64_t dims[3], uint32_t* shift, uint32_t mn[3])
     }
 }
 
+// Device memory that a grid's upload goes through.
+constexpr uint64_t kGridStagingBytes = 256ull << 20;
+
 uint64_t grid_footprint(const uint64_t dims[3]) {
     uint64_t nbricks = 1;
     for (int i = 0; i < 3; ++i) nbricks *= (dims[i] + kBrick - 1) / kBrick;
@@ -309,20 +312,31 @@ int xd_volume_from_grid(xd_context* ctx, const void* rgba8, uint64_t dim_x, uint
     const uint32_t dims32[3] = {(uint32_t)dim_x, (uint32_t)dim_y, (uint32_t)dim_z};
     uint32_t* staging = nullptr;
     const uint64_t layer_texels = dim_x * dim_y;
-    if ((e = hipMalloc(&v->d_bricks, brick_bytes)) != hipSuccess || (e = hipMalloc(&v->d_occ, nbricks)) != hipSuccess ||
-        (e = hipMalloc(&staging, layer_texels * kBrick * sizeof(uint32_t))) != hipSuccess) {
-        if (staging) (void)hipFree(staging);
+    if ((e = hipMalloc(&v->d_bricks, brick_bytes)) != hipSuccess || (e = hipMalloc(&v->d_occ, nbricks)) != hipSuccess) {
         xd_volume_free(v);
         return fail_hip(e, "grid allocation");
     }
+    // several brick layers a copy: a copy of pageable memory costs about 0.1 ms
+    // beside its bytes.  Less where the device has no room for it.
+    uint64_t layers_at_once = kBrick;
+    while (layers_at_once < dim_z && layers_at_once * 2 * layer_texels * sizeof(uint32_t) <= kGridStagingBytes)
+        layers_at_once *= 2;
+    while ((e = hipMalloc(&staging, layers_at_once * layer_texels * sizeof(uint32_t))) != hipSuccess) {
+        if (layers_at_once == kBrick) {
+            xd_volume_free(v);
+            return fail_hip(e, "grid allocation");
+        }
+        (void)hipGetLastError();
+        layers_at_once /= 2;
+    }
     v->bytes = brick_bytes + nbricks;
     const uint8_t* src = static_cast<const uint8_t*>(rgba8);
-    for (uint32_t bz = 0; bz < v->nb[2]; ++bz) {
-        const uint64_t z0 = (uint64_t)bz * kBrick;
-        const uint32_t layers = (uint32_t)std::min<uint64_t>(kBrick, dim_z - z0);
+    for (uint64_t z0 = 0; z0 < dim_z; z0 += layers_at_once) {
+        const uint32_t layers = (uint32_t)std::min<uint64_t>(layers_at_once, dim_z - z0);
         e = hipMemcpyAsync(staging, src + z0 * layer_texels * 4, layers * layer_texels * 4, hipMemcpyHostToDevice,
                            ctx->stream);
-        if (e == hipSuccess) e = launch_brick_layer(staging, layers, bz, v->d_bricks, v->d_occ, dims32, v->nb, ctx->stream);
+        if (e == hipSuccess)
+            e = launch_bricks(staging, layers, (uint32_t)(z0 / kBrick), v->d_bricks, v->d_occ, dims32, v->nb, ctx->stream);
         if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
         if (e != hipSuccess) {
             (void)hipFree(staging);
