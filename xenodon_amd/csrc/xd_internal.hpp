@@ -44,6 +44,7 @@ constexpr uint32_t kTopLevels = 4;
 constexpr uint32_t kTableLevel = 8;
 constexpr uint64_t kTableCells = 1ull << (3 * kTableLevel);
 constexpr uint64_t kTableBytes = kTableCells * 8;
+constexpr uint32_t kRecWords = 12;  // words of an internal node's record (RenderParams::rec)
 
 // Everything one traversal launch needs; passed by value as the kernel
 // argument (kernarg segment), so a launch needs no device-side setup.
@@ -83,6 +84,13 @@ struct RenderParams {
     uint32_t empty_start;  // wide tags: child indices from here on are empty leaves (else 0xFFFFFFFF)
     uint32_t leaf_base;    // tagged layout: first leaf; rope k of leaf l >= leaf_base is word
                            // leaf_base*8 + k*(node_count - leaf_base) + (l - leaf_base) of cw
+    // records of the internal nodes, or null (DAGs and what else the host
+    // derives): kRecWords words each, {first internal child, masks of the
+    // internal children (bits 0..7), the leaves with colour (8..15) and the
+    // internal children without internal children (16..23), 0, 0, the children's
+    // RGB (0 for all but leaves)}.  A node's internal children have
+    // consecutive indices, so one index and a mask name them all.
+    const uint4* rec;
     uint32_t xcd_chunks;  // plain launches: block runs per XCD (0: hardware order)
     unsigned long long* words;  // word counter (instrumented variant only)
 };

@@ -15,7 +15,7 @@
 //                   them per block
 //   k_oct_number    scans the block's sums, gives each child its word
 //   k_oct_emit      scans again (cheaper than keeping 12 bytes a node) and
-//                   writes child words, colours, depths and ropes
+//                   writes child words, records, colours, depths and ropes
 // The passes read the nodes' 40 bytes and, scattered over nearby nodes, their
 // children's words: for a tree of 1.3 million nodes (192x137x192 voxels) 59 us
 // with the checks, 24 and 30 us, about 1 TB/s each, then 53 us for the 128 MiB
@@ -262,7 +262,8 @@ __global__ __launch_bounds__(kOctBlock) void k_oct_emit(const uint2* __restrict_
                                                         const uint4* __restrict__ base, const uint4* __restrict__ top,
                                                         OctBases B, uint32_t empty_tag, uint32_t index_mask,
                                                         const uint32_t* __restrict__ words, uint32_t* __restrict__ cw,
-                                                        uint32_t* __restrict__ meta, OctFlags* flags) {
+                                                        uint4* __restrict__ rec, uint32_t* __restrict__ meta,
+                                                        OctFlags* flags) {
     const uint64_t i = (uint64_t)blockIdx.x * kOctBlock + threadIdx.x;
     uint2 cm = make_uint2(0, kLeafMask);  // {colour, is_leaf_depth}
     if (i < n) cm = raw[i * 5 + 4];
@@ -288,6 +289,18 @@ __global__ __launch_bounds__(kOctBlock) void k_oct_emit(const uint2* __restrict_
         uint4* const out = reinterpret_cast<uint4*>(cw + (uint64_t)id * 8);
         out[0] = make_uint4(w[0], w[1], w[2], w[3]);
         out[1] = make_uint4(w[4], w[5], w[6], w[7]);
+        uint32_t low = 0;  // internal children without internal children
+#pragma unroll
+        for (uint32_t k = 0; k < 8; ++k)
+            if (inner_mask(m) >> k & 1u && inner_mask(masks[c[k]]) == 0) low |= 0x10000u << k;
+        uint32_t col[8];  // 0 but for leaves with colour
+#pragma unroll
+        for (uint32_t k = 0; k < 8; ++k)
+            col[k] = colour_mask(m) >> k & 1u ? raw[(uint64_t)c[k] * 5 + 4].x & 0xFFFFFFu : 0u;
+        uint4* const r = rec + (uint64_t)id * kRecWords / 4;
+        r[0] = make_uint4(first[0], (m & 0xFFFFu) | low, 0, 0);
+        r[1] = make_uint4(col[0], col[1], col[2], col[3]);
+        r[2] = make_uint4(col[4], col[5], col[6], col[7]);
     } else if (id >= B.leaf_base) {  // six ropes; a leaf root has no planes
         const uint64_t nl = n - B.leaf_base, at = (uint64_t)B.leaf_base * 8 + (id - B.leaf_base);
 #pragma unroll
@@ -397,6 +410,10 @@ bool derive_layout_on_device(xd_volume* v, const uint32_t* w, uint64_t n, bool w
         B.empty_base = B.leaf_base + count[1] + f.total[1];
         const bool depth_bits = !wide && n <= (uint64_t)kRopeIndexMask + 1 && f.depth < 32;
         const uint32_t index_mask = depth_bits ? kRopeIndexMask : wide ? kWideIndexMask : kIndexMask;
+        // the records follow the leaves' ropes, in the two words a leaf that six
+        // planes leave of the eight the footprint counts
+        const uint64_t rec_at = (rope_plane_words(n, B.leaf_base) + 3) & ~3ull;
+        if (!root_leaf && rec_at + (uint64_t)kRecWords * B.leaf_base > n * 8) break;
         if ((e = hipMalloc(&v->d_cw, n * 8 * sizeof(uint32_t))) != hipSuccess ||
             (e = hipMalloc(&v->d_meta, n * 2 * sizeof(uint32_t))) != hipSuccess ||
             (e = hipMalloc(&v->d_table, kTableBytes)) != hipSuccess)
@@ -404,7 +421,8 @@ bool derive_layout_on_device(xd_volume* v, const uint32_t* w, uint64_t n, bool w
         hipLaunchKernelGGL(k_oct_number, dim3(blocks), dim3(kOctBlock), 0, s, raw, (uint32_t)n, masks, base, d_top, B,
                            v->root_tag, empty_tag, depth_bits ? 1u : 0u, words);
         hipLaunchKernelGGL(k_oct_emit, dim3(blocks), dim3(kOctBlock), 0, s, raw, (uint32_t)n, masks, base, d_top, B,
-                           empty_tag, index_mask, words, v->d_cw, v->d_meta, flags);
+                           empty_tag, index_mask, words, v->d_cw, reinterpret_cast<uint4*>(v->d_cw + rec_at), v->d_meta,
+                           flags);
         if ((e = hipGetLastError()) != hipSuccess ||
             (e = launch_start_table(v->d_cw, v->root_tag, index_mask, &flags->twice, v->d_table, s)) != hipSuccess ||
             (e = hipMemcpyAsync(&f, flags, sizeof(f), hipMemcpyDeviceToHost, s)) != hipSuccess ||
@@ -419,6 +437,7 @@ bool derive_layout_on_device(xd_volume* v, const uint32_t* w, uint64_t n, bool w
         v->empty_tag = empty_tag;
         v->empty_start = wide ? B.empty_base : 0xFFFFFFFFu;
         v->leaf_base = B.leaf_base;
+        v->rec_at = root_leaf ? 0 : rec_at;
         done = true;
     } while (false);
     if (e != hipSuccess) (void)hipGetLastError();  // reported by the host path if it fails as well

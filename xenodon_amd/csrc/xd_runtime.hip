@@ -126,6 +126,7 @@ void fill_params(RenderParams& p, const xd_volume* vol, int traversal, const xd_
         p.node_count = (uint32_t)vol->node_count;
         p.depth_exact = vol->depth_exact;
         p.leaf_base = vol->leaf_base;
+        p.rec = vol->rec_at ? reinterpret_cast<const uint4*>(vol->d_cw + vol->rec_at) : nullptr;
     }
 }
 

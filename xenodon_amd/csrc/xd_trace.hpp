@@ -283,6 +283,8 @@ __device__ __forceinline__ f3 svo_pixel(const RenderParams& p, f3 rd, uint32_t* 
         float t0, t1;
         aabb_intersect(splat(1.0f), splat(2.0f), ro, rd, t0, t1);
         ro = add(ro, smul(gmax(t0, 0.0f), rd));
+        if (TAGGED && !COUNT && p.rec)
+            return fast_esvo_rec(p.rec, p.leaf_base, p.cap, p.stack_slots, ro, rd, stk_a, stk_tmax);
         if (TAGGED && !COUNT) return fast_esvo(fs, p.cap, p.stack_slots, ro, rd, stk_a,
                                                 stk_tmax);
         if (TAGGED) return ref_esvo<COUNT>(TaggedNodes{p.cw, p.meta, p.node_count, p.index_mask, p.leaf_base}, p.cap, p.stack_slots, ro, rd, stk_a, stk_tmax,
@@ -291,6 +293,8 @@ __device__ __forceinline__ f3 svo_pixel(const RenderParams& p, f3 rd, uint32_t* 
     }
     const f3 ro = p.cam.translation;
     if (TRAV == 3) {  // svo-df
+        if (TAGGED && !COUNT && p.rec)
+            return fast_df_rec(p.rec, p.leaf_base, p.cap, ro, rd, stk_a, stk_b);
         if (TAGGED && !COUNT)  // depth-field handling fixed per tree (a uniform choice)
             return p.depth_exact ? fast_df<true>(fs, p.cap, p.stack_slots, ro, rd, stk_a, stk_b)
                                  : fast_df<false>(fs, p.cap, p.stack_slots, ro, rd, stk_a, stk_b);
