@@ -44,6 +44,9 @@ constexpr uint32_t kTopLevels = 4;
 constexpr uint32_t kTableLevel = 8;
 constexpr uint64_t kTableCells = 1ull << (3 * kTableLevel);
 constexpr uint64_t kTableBytes = kTableCells * 8;
+// The entry's second word: the level, and whether the node is internal with only
+// leaves for children and has a record.
+constexpr uint32_t kTableLevelMask = 0xFFu, kTableLowNode = 0x100u;
 constexpr uint32_t kRecWords = 12;  // words of an internal node's record (RenderParams::rec)
 
 // Everything one traversal launch needs; passed by value as the kernel

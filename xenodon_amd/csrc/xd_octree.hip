@@ -314,12 +314,15 @@ __global__ __launch_bounds__(kOctBlock) void k_oct_emit(const uint2* __restrict_
 // One cell of the start table a thread: the walk of build_start_table.
 // stop: null, or a word that says, when set, that the child words are no tree's.
 __global__ __launch_bounds__(256) void k_start_table(const uint32_t* __restrict__ cw, uint32_t root_tag,
-                                                     uint32_t index_mask, const uint32_t* stop,
-                                                     uint2* __restrict__ table) {
+                                                     uint32_t index_mask, const uint4* __restrict__ rec,
+                                                     const uint32_t* stop, uint2* __restrict__ table) {
     if (stop && *stop) return;
     const uint32_t cell = blockIdx.x * 256 + threadIdx.x;
     constexpr uint32_t L = kTableLevel, side = (1u << L) - 1u;
-    const uint32_t x = cell & side, y = cell >> L & side, z = cell >> (2 * L);
+    // cells in the table's order (table_cell)
+    const uint32_t brick = cell >> 6;
+    const uint32_t x = (brick << 2 & side) | (cell & 3u), y = (brick >> (L - 2) << 2 & side) | (cell >> 2 & 3u),
+                   z = (brick >> (2 * (L - 2)) << 2) | (cell >> 4 & 3u);
     uint32_t word = root_tag, level = 0;
     while (!(word & kTagLeaf) && level < L) {
         const uint32_t s = L - 1 - level;
@@ -327,15 +330,17 @@ __global__ __launch_bounds__(256) void k_start_table(const uint32_t* __restrict_
         word = cw[(uint64_t)(word & index_mask) * 8 + k];
         ++level;
     }
+    if (!(word & kTagLeaf) && rec && (rec[(uint64_t)(word & index_mask) * (kRecWords / 4)].y & 0xFFu) == 0)
+        level |= kTableLowNode;
     table[cell] = make_uint2(word, level);
 }
 
 }  // namespace
 
-hipError_t launch_start_table(const uint32_t* cw, uint32_t root_tag, uint32_t index_mask, const uint32_t* stop,
-                              uint2* table, hipStream_t s) {
+hipError_t launch_start_table(const uint32_t* cw, uint32_t root_tag, uint32_t index_mask, const uint4* rec,
+                              const uint32_t* stop, uint2* table, hipStream_t s) {
     hipLaunchKernelGGL(k_start_table, dim3((uint32_t)(kTableCells / 256)), dim3(256), 0, s, cw, root_tag, index_mask,
-                       stop, table);
+                       rec, stop, table);
     return hipGetLastError();
 }
 
@@ -418,13 +423,13 @@ bool derive_layout_on_device(xd_volume* v, const uint32_t* w, uint64_t n, bool w
             (e = hipMalloc(&v->d_meta, n * 2 * sizeof(uint32_t))) != hipSuccess ||
             (e = hipMalloc(&v->d_table, kTableBytes)) != hipSuccess)
             break;
+        uint4* const rec = reinterpret_cast<uint4*>(v->d_cw + rec_at);
         hipLaunchKernelGGL(k_oct_number, dim3(blocks), dim3(kOctBlock), 0, s, raw, (uint32_t)n, masks, base, d_top, B,
                            v->root_tag, empty_tag, depth_bits ? 1u : 0u, words);
         hipLaunchKernelGGL(k_oct_emit, dim3(blocks), dim3(kOctBlock), 0, s, raw, (uint32_t)n, masks, base, d_top, B,
-                           empty_tag, index_mask, words, v->d_cw, reinterpret_cast<uint4*>(v->d_cw + rec_at), v->d_meta,
-                           flags);
+                           empty_tag, index_mask, words, v->d_cw, rec, v->d_meta, flags);
         if ((e = hipGetLastError()) != hipSuccess ||
-            (e = launch_start_table(v->d_cw, v->root_tag, index_mask, &flags->twice, v->d_table, s)) != hipSuccess ||
+            (e = launch_start_table(v->d_cw, v->root_tag, index_mask, root_leaf ? nullptr : rec, &flags->twice, v->d_table, s)) != hipSuccess ||
             (e = hipMemcpyAsync(&f, flags, sizeof(f), hipMemcpyDeviceToHost, s)) != hipSuccess ||
             (e = hipStreamSynchronize(s)) != hipSuccess)
             break;

@@ -534,7 +534,7 @@ int xd_volume_from_svo(xd_context* ctx, const void* nodes, uint64_t node_count, 
         const uint32_t root_ld = w[9], root_col = w[8];
         v->root_tag = (root_ld & kLeafMask) ? (kTagLeaf | ((root_col & 0xFFFFFFu) ? 0u : v->empty_tag)) : 0u;
         if ((e = hipMalloc(&v->d_table, kTableBytes)) != hipSuccess ||
-            (e = launch_start_table(v->d_cw, v->root_tag, v->index_mask, nullptr, v->d_table, ctx->stream)) != hipSuccess ||
+            (e = launch_start_table(v->d_cw, v->root_tag, v->index_mask, nullptr, nullptr, v->d_table, ctx->stream)) != hipSuccess ||
             (e = hipStreamSynchronize(ctx->stream)) != hipSuccess) {
             xd_volume_free(v);
             return fail_hip(e, "octree upload");

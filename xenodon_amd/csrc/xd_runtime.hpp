@@ -111,10 +111,11 @@ bool octree_depths_exact(const uint32_t* w, uint64_t n, bool tree);
 // child words for at most L levels, so any tree, cyclic ones included, gives
 // a table.
 void build_start_table(const uint32_t* child_w, uint32_t root_tag, uint32_t index_mask, uint2* table);
-// The same table built on the device, from the device form of child_w.  stop:
+// The device's table, built there from the device form of child_w: the same
+// entries in the order of table_cell, with kTableLowNode from rec (or null).  stop:
 // null, or a device word that, if set, keeps the table unwritten.
-hipError_t launch_start_table(const uint32_t* cw, uint32_t root_tag, uint32_t index_mask, const uint32_t* stop,
-                              uint2* table, hipStream_t s);
+hipError_t launch_start_table(const uint32_t* cw, uint32_t root_tag, uint32_t index_mask, const uint4* rec,
+                              const uint32_t* stop, uint2* table, hipStream_t s);
 // Derives v's tagged layout and start table on the device from n .svo nodes in
 // host memory, and sets everything of v that depends on them.  False if the
 // tree or the device memory does not allow it (see xd_octree.hip); v is as it

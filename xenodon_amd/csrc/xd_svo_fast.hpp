@@ -92,9 +92,18 @@ __device__ __forceinline__ uint32_t colour_if(const FastSvo& s, uint32_t node, u
 // bit (22 - l) of floor(p * 2^23); p < 0 (or NaN) fails every comparison and
 // p >= 1 passes every one.
 __device__ __forceinline__ uint32_t level_bits(float p) {
-    if (!(p > 0.0f)) return 0u;
-    if (!(p < 1.0f)) return (1u << 23) - 1u;
-    return (uint32_t)(p * 8388608.0f);
+    // the conversion gives 0 for negative numbers and NaN, and the largest word
+    // for numbers beyond it
+    uint32_t b;
+    asm("v_cvt_u32_f32 %0, %1" : "=v"(b) : "v"(p * 8388608.0f));
+    return min(b, (1u << 23) - 1u);
+}
+
+// Index of cell (x, y, z) in the start table: 4x4x4 cells together, 512 B, as
+// the rays of a tile walk neighbouring cells along any axis.
+__device__ __forceinline__ uint32_t table_cell(uint32_t x, uint32_t y, uint32_t z) {
+    constexpr uint32_t b = kTableLevel - 2;
+    return (((z >> 2) << (2 * b) | (y >> 2) << b | (x >> 2)) << 6) | (z & 3u) << 4 | (y & 3u) << 2 | (x & 3u);
 }
 
 // svo_naive.comp:8-27 with tagged pointers.  `tag` returns the found node's
@@ -111,10 +120,10 @@ __device__ __forceinline__ uint32_t fast_find(const FastSvo& s, f3 pos, f3& base
     if (s.table) {
         const uint32_t bx = level_bits(pos.x), by = level_bits(pos.y), bz = level_bits(pos.z);
         constexpr uint32_t sh = 23u - kTableLevel;
-        const uint2 e = s.table[((bz >> sh) << (2 * kTableLevel)) | ((by >> sh) << kTableLevel) | (bx >> sh)];
+        const uint2 e = s.table[table_cell(bx >> sh, by >> sh, bz >> sh)];
         index = e.x & s.index_mask;
         tag = e.x;
-        level = e.y;
+        level = e.y & kTableLevelMask;
         extent = __builtin_ldexpf(1.0f, -(int)level);
         const uint32_t c = 23u - level;  // 32-bit shifts: level >= 1 here, or the bits are unused
         offset = level == 0 ? splat(0.0f)
@@ -138,8 +147,18 @@ __device__ __forceinline__ uint32_t fast_find(const FastSvo& s, f3 pos, f3& base
     }
 }
 
-// svo_naive.comp:29-71
-__device__ __forceinline__ f3 fast_naive(const FastSvo& s, uint64_t cap, f3 ro, f3 rd) {
+// svo_naive.comp:29-71.  A step's position depends on the box of the leaf before
+// it, so a ray is one chain of loads; what is not on it is kept off it:
+//  * the start table says where a cell's node has only leaves for children.
+//    Such a child's box follows from the position's bits, so the step goes on
+//    without waiting for its word;
+//  * a leaf's colour is added one step late, while the next step's table entry
+//    is on its way;
+//  * a step that stays in its cell keeps the entry (rays almost parallel to a
+//    plane advance by min_step for thousands of steps).
+// Plain 1080p frames of a 512x361x512 volume (outside / over it / inside): 0.70
+// / 0.63 / 1.96 -> 0.52 / 0.50 / 1.50 ms, the table in 4x4x4 cells included.
+__device__ __forceinline__ f3 fast_naive(const FastSvo& s, const uint4* __restrict__ rec, uint64_t cap, f3 ro, f3 rd) {
     const float min_step = 0.00001f;
     f3 rrd = divv(splat(1.0f), rd);
     f3 bias = mul(rrd, ro);
@@ -153,23 +172,52 @@ __device__ __forceinline__ f3 fast_naive(const FastSvo& s, uint64_t cap, f3 ro, 
     float t = t_min + min_step;
     const uint32_t cap32 = cap32_of(cap);
     uint32_t it = 0;
+    uint32_t cell = ~0u;
+    uint2 e = make_uint2(0, 0);
+    uint32_t pend_col = 0;  // the last leaf's term, added at the next step
+    float pend_w = 0.0f;
     while (t < t_max) {
         if (++it > cap32) break;
-        f3 pt = add(smul(t, rd), ro);
-        f3 offset;
-        float side;
-        uint32_t tag;
-        uint32_t node = fast_find(s, pt, offset, side, tag);
+        const f3 pt = add(smul(t, rd), ro);
+        const uint32_t bx = level_bits(pt.x), by = level_bits(pt.y), bz = level_bits(pt.z);
+        constexpr uint32_t sh = 23u - kTableLevel;
+        const uint32_t at = table_cell(bx >> sh, by >> sh, bz >> sh);
+        if (at != cell) {
+            e = s.table[at];
+            cell = at;
+        }
+        total = add(total, muls(unorm_rgb(pend_col), pend_w));  // +0 the first time
+        uint32_t word = e.x, level = e.y & kTableLevelMask;
+        const uint32_t* colour = s.meta;  // of the leaf, or null for none
+        if (e.y & kTableLowNode) {
+            const uint32_t k = (bx >> (sh - 1) & 1u) << 2 | (by >> (sh - 1) & 1u) << 1 | (bz >> (sh - 1) & 1u);
+            colour = reinterpret_cast<const uint32_t*>(rec) + (uint64_t)(word & s.index_mask) * kRecWords + 4u + k;
+            ++level;
+        } else {
+            while (!(word & kTagLeaf) && level <= kMaxLevels) {
+                const uint32_t d = 22u - min(level, 22u);
+                const uint32_t k = (bx >> d & 1u) << 2 | (by >> d & 1u) << 1 | (bz >> d & 1u);
+                word = cw_at(s, word & s.index_mask, k);
+                ++level;
+            }
+            colour = empty_leaf(s, word) ? nullptr : s.meta + (word & s.index_mask);
+        }
+        // 1 + the leaf's corner is its leading bits after the point
+        const uint32_t keep = ~0u << (23u - level);
+        const f3 offset = mk(u2f(0x3F800000u | (bx & keep)) - 1.0f, u2f(0x3F800000u | (by & keep)) - 1.0f,
+                             u2f(0x3F800000u | (bz & keep)) - 1.0f);
+        const float side = __builtin_ldexpf(1.0f, -(int)level);
         f3 node_min = sub(mul(offset, rrd), bias);
         f3 node_max = sub(mul(add(offset, splat(side)), rrd), bias);
         float u_min = max_elem(vmin(node_min, node_max));
         float u_max = min_elem(vmax(node_min, node_max));
         u_min = gmax(u_min, 0.0f);
-        float step = gmax(u_max - u_min, min_step);
+        const float step = gmax(u_max - u_min, min_step);
         t = t + step;
-        total = add(total, muls(unorm_rgb(colour_if(s, node, tag)), step));
+        pend_col = colour ? *colour : 0u;
+        pend_w = step;
     }
-    return total;
+    return add(total, muls(unorm_rgb(pend_col), pend_w));
 }
 
 __device__ __forceinline__ uint32_t pick8(const uint4& lo, const uint4& hi, uint32_t ci) {

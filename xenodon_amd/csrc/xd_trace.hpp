@@ -302,7 +302,7 @@ __device__ __forceinline__ f3 svo_pixel(const RenderParams& p, f3 rd, uint32_t* 
         return ref_df<COUNT>(RawNodes{p.nodes, p.node_count}, p.cap, p.stack_slots, ro, rd, stk_a, stk_b, words);
     }
     if (TRAV == 1) {  // svo-naive
-        if (TAGGED && !COUNT) return fast_naive(fs, p.cap, ro, rd);
+        if (TAGGED && !COUNT) return fast_naive(fs, p.rec, p.cap, ro, rd);
         if (TAGGED) return ref_naive<COUNT>(TaggedNodes{p.cw, p.meta, p.node_count, p.index_mask, p.leaf_base}, p.cap, ro, rd, words);
         return ref_naive<COUNT>(RawNodes{p.nodes, p.node_count}, p.cap, ro, rd, words);
     }
