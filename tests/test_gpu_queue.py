@@ -49,3 +49,32 @@ def test_queue_sizes_match_plain_renders(env, travs, class_kernels, waves, grab)
             assert np.array_equal(v[4].download(), ref), (n, W, Hh, "static")
             v[4].free()
     b.free()
+
+
+@pytest.mark.parametrize("order", [0, 2, 3, 4])
+@pytest.mark.parametrize("tile_w,rpl", [(8, 1), (16, 2), (32, 4)])
+def test_every_tile_is_dealt(env, order, tile_w, rpl):
+    """Every pixel of views cut into whole, narrow and low squares is rendered: the frames are black before, and
+    every ray inside this volume is lit."""
+    ctx, _, _ = env
+    grid = H.random_grid((24, 24, 24), density=1.0, seed=3)
+    vol = ctx.grid_volume(grid)
+    away = abi.make_camera(*H.look_at((0.5, 0.5, 3.0), (0.5, 0.5, 9.0)))
+    views = []
+    for k, (W, Hh) in enumerate([(8, 8), (65, 8), (8, 65), (129, 57), (520, 24), (24, 520), (333, 222), (1, 700)]):
+        fr = ctx.frame(W, Hh)
+        uni = abi.make_uniforms(W, Hh, [24] * 3, emission=2.0)
+        ctx.render(vol, abi.DDA, away, uni, fr)
+        assert not fr.download()[..., :3].any()
+        views.append((vol, abi.DDA, abi.make_camera(*H.look_at((0.5, 0.45, 0.55), (0.2 + 0.1 * k, 0.5, 0.1))), uni, fr))
+    b = ctx.batch()
+    b.set_tuning([tile_w] * 5, interleave=order, rays_per_lane=[rpl] * 5)
+    b.set_views(views)
+    b.render()
+    for v in views:
+        got = v[4].download()
+        assert got[..., :3].any(-1).all()
+        assert np.array_equal(got, ctx.render_image(*v[:4])[0])
+        v[4].free()
+    b.free()
+    vol.free()

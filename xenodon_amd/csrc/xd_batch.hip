@@ -32,6 +32,56 @@
 
 namespace xd {
 
+// How a view's wave tiles go to the queues (orders 0, 2, 3, 4): cut into squares
+// of sw x sh tile groups (a group: rpl rows of tiles), dealt to the queues in
+// turn, row by row; within a square the groups are row-major.  Neighbouring
+// squares thus run on different XCDs, as the plain launches' blocks do, and no
+// XCD is left with a view's costly part: 1080p frames of one traversal, batched
+// alone, took 0.47 (dda), 0.48 (svo-naive) and 0.52 ms (svo-rope) with a band of
+// the view to each XCD, 0.37, 0.36 and 0.39 so.
+struct TileDeal {
+    uint32_t tiles_x, rows, rpl, sw, sh;  // rows: groups
+    __host__ __device__ uint32_t squares_x() const { return (tiles_x + sw - 1) / sw; }
+    __host__ __device__ uint32_t squares_y() const { return (rows + sh - 1) / sh; }
+    // Entries of queue k in the first r rows of squares, all of height sh.
+    __host__ __device__ uint32_t above(uint32_t r, uint32_t k) const {
+        const uint32_t nx = squares_x(), narrow = nx * sw - tiles_x;  // what the last column lacks
+        const uint32_t n = (r * nx + kQueues - 1 - k) / kQueues;      // squares k, k + 8, ...
+        uint32_t last = 0;                                            // of them in the last column
+        for (uint32_t p = 0; p < kQueues && p < r; ++p)  // the rows p, p + 8, ... end in the same queue
+            if ((p * nx + nx - 1) % kQueues == k) last += (r - p + kQueues - 1) / kQueues;
+        return (n * sw - last * narrow) * sh * rpl;
+    }
+    __host__ __device__ uint32_t total(uint32_t k) const {
+        const uint32_t r = squares_y() - 1, nx = squares_x(), h = rows - r * sh;
+        uint32_t w = 0;
+        for (uint32_t c = (k + kQueues - r * nx % kQueues) % kQueues; c < nx; c += kQueues)
+            w += c + 1 < nx ? sw : tiles_x - c * sw;
+        return above(r, k) + w * h * rpl;
+    }
+};
+
+uint32_t square_width(uint32_t order) { return order == 3 ? 4u : order == 4 ? 16u : 8u; }
+uint32_t square_height(uint32_t order) { return order == 0 ? 1u : square_width(order); }
+
+// The tile table of the views, one entry a thread (blockIdx.y: the view); view
+// i's entries of queue k begin at first[k].  For 1.3 million tiles (40 views of
+// 1920x1080) the host had taken 1.3 ms to write and upload the same table.
+__global__ __launch_bounds__(256) void k_deal_tiles(const BatchView* __restrict__ views, uint32_t sw, uint32_t sh,
+                                                    uint32_t* __restrict__ tiles) {
+    const BatchView& V = views[blockIdx.y];
+    const TileDeal D{V.tiles_x, V.rows, V.rpl, sw, sh};
+    const uint32_t e = blockIdx.x * 256 + threadIdx.x;
+    if (e >= D.tiles_x * D.rows * D.rpl) return;
+    const uint32_t tx = e % D.tiles_x, y = e / D.tiles_x, ty = y / D.rpl;
+    const uint32_t sx = tx / sw, sy = ty / sh, nx = D.squares_x(), k = (sy * nx + sx) % kQueues;
+    const uint32_t w = min(sw, D.tiles_x - sx * sw), h = min(sh, D.rows - sy * sh);
+    // the squares of this row before this one are whole, each eighth of them in its queue
+    const uint32_t at = V.first[k] + D.above(sy, k) + sx / kQueues * sw * h * D.rpl +
+                        ((ty - sy * sh) * w + (tx - sx * sw)) * D.rpl + y % D.rpl;
+    tiles[at] = blockIdx.y << 20 | e;
+}
+
 __global__ void k_batch_reset(uint32_t* counters) {
     if (threadIdx.x < kClasses * kQueues) counters[threadIdx.x * kCounterStride] = 0;
 }
@@ -368,15 +418,16 @@ void deal_by_affinity(std::vector<std::vector<uint32_t>>& q) {
 // The view and tile tables of a launch, built on the host.
 struct HostTables {
     std::vector<BatchView> views;
-    std::vector<uint32_t> tiles;
+    std::vector<uint32_t> tiles;  // empty where the device deals them (k_deal_tiles)
+    uint32_t total_tiles, most_tiles;  // of all views, of one view
     uint32_t qbeg[kClasses * kQueues + 1];
     BatchClasses cls;  // grid[c] = 1 if kernel c has tiles; slots[c] its LDS stack stride
     uint64_t total_rays;
 };
 
 // Builds the view and tile tables of n views under a tuning.  Tiles are
-// grouped by class, and within a class dealt into kQueues ranges by the band
-// of their view they lie in.
+// grouped by class, and within a class dealt into kQueues ranges: in squares by
+// the device (TileDeal), or by the band of their view they lie in.
 // keep_mixed: a batch of one traversal still runs the all-traversal kernel
 // when the tuning says so (the autotuner times one traversal's views on the
 // kernel the whole batch will run).
@@ -393,6 +444,9 @@ int build_tables(const xd_view* views, uint32_t n, const xd_batch_tuning& tuning
     std::vector<Group> groups;
     BatchClasses cls{};
     T.total_rays = 0;
+    T.most_tiles = 0;
+    const uint32_t order = tuning.interleave, sw = square_width(order), sh = square_height(order);
+    const bool interleaved = order == 1 || order == 5;
     for (uint32_t i = 0; i < n; ++i) {
         const xd_view& v = views[i];
         BatchView& B = bv[i];
@@ -412,8 +466,9 @@ int build_tables(const xd_view* views, uint32_t n, const xd_batch_tuning& tuning
         const uint32_t c = (uint32_t)v.traversal;
         cls.slots[c] = std::max(cls.slots[c], batch_view_slots(B));
         cls.grid[c] = 1;
-        const uint32_t order = tuning.interleave;
-        if (order == 1 || order == 5) {
+        B.rows = big_y;
+        T.most_tiles = std::max(T.most_tiles, big_y * rpl * B.tiles_x);
+        if (interleaved) {
             // views of one volume, traversal, size and tile shape form a group
             // whose tiles are dealt together below
             const uint64_t key[6] = {(uint64_t)(uintptr_t)v.volume, (uint64_t)c, W, H, B.tw_shift, B.rpl};
@@ -421,25 +476,12 @@ int build_tables(const xd_view* views, uint32_t n, const xd_batch_tuning& tuning
             while (g < groups.size() && memcmp(groups[g].key, key, sizeof key) != 0) ++g;
             if (g == groups.size()) groups.push_back({{key[0], key[1], key[2], key[3], key[4], key[5]}, {}, B.tiles_x, big_y});
             groups[g].views.push_back(i);
-        } else {
-            // squares of sq x sq groups of rows (sq = 1: plain rows),
-            // row-major within each band's squares
-            const uint32_t sq = order == 2 ? 8u : order == 3 ? 4u : order == 4 ? 16u : 1u;
-            for (uint32_t ty0 = 0; ty0 < big_y; ty0 += sq) {
-                const uint32_t band = (uint32_t)((uint64_t)ty0 * kQueues / big_y);
-                const uint32_t ty1 = std::min(big_y, ty0 + sq);
-                for (uint32_t tx0 = 0; tx0 < B.tiles_x; tx0 += sq)
-                    for (uint32_t ty = ty0; ty < ty1; ++ty)
-                        for (uint32_t tx = tx0; tx < std::min(B.tiles_x, tx0 + sq); ++tx)
-                            for (uint32_t r = 0; r < rpl; ++r)
-                                q[c * kQueues + band].push_back((i << 20) | ((ty * rpl + r) * B.tiles_x + tx));
-            }
         }
         T.total_rays += (uint64_t)W * H;
     }
     // interleaved: the same tile of every view of a group, one after another
     // (order 5: in squares of 8 x 8 tiles)
-    const uint32_t gsq = tuning.interleave == 5 ? 8u : 1u;
+    const uint32_t gsq = order == 5 ? 8u : 1u;
     for (const auto& G : groups)
         for (uint32_t ty0 = 0; ty0 < G.tiles_y; ty0 += gsq) {
             const uint32_t band = (uint32_t)((uint64_t)ty0 * kQueues / G.tiles_y);
@@ -472,21 +514,61 @@ int build_tables(const xd_view* views, uint32_t n, const xd_batch_tuning& tuning
     }
     for (uint32_t i = 0; i < n; ++i)
         bv[i].p.lds_slots = std::max<uint32_t>(cls.slots[per_class ? bv[i].traversal : kClasses], 1);
-    if (!per_class && tuning.mix_classes == 2) deal_by_affinity(q);
+    const bool affinity = !per_class && tuning.mix_classes == 2;
     uint64_t total = 0;
-    for (uint32_t k = 0; k < kClasses * kQueues; ++k) {
-        T.qbeg[k] = (uint32_t)total;
-        total += q[k].size();
+    T.tiles.clear();
+    if (interleaved || affinity) {
+        // orders that the host deals: a band of each view to a queue
+        for (uint32_t i = 0; i < n && !interleaved; ++i) {
+            const BatchView& B = bv[i];
+            for (uint32_t ty0 = 0; ty0 < B.rows; ty0 += sh) {
+                const uint32_t band = (uint32_t)((uint64_t)ty0 * kQueues / B.rows);
+                for (uint32_t tx0 = 0; tx0 < B.tiles_x; tx0 += sw)
+                    for (uint32_t ty = ty0; ty < std::min(B.rows, ty0 + sh); ++ty)
+                        for (uint32_t tx = tx0; tx < std::min(B.tiles_x, tx0 + sw); ++tx)
+                            for (uint32_t r = 0; r < B.rpl; ++r)
+                                q[B.traversal * kQueues + band].push_back((i << 20) | ((ty * B.rpl + r) * B.tiles_x + tx));
+            }
+        }
+        if (affinity) deal_by_affinity(q);
+        for (uint32_t k = 0; k < kClasses * kQueues; ++k) {
+            T.qbeg[k] = (uint32_t)total;
+            total += q[k].size();
+        }
+    } else {
+        uint64_t size[kClasses * kQueues] = {};
+        for (const BatchView& B : bv)
+            for (uint32_t k = 0; k < kQueues; ++k)
+                size[B.traversal * kQueues + k] += TileDeal{B.tiles_x, B.rows, B.rpl, sw, sh}.total(k);
+        uint32_t at[kClasses * kQueues];
+        for (uint32_t k = 0; k < kClasses * kQueues; ++k) {
+            T.qbeg[k] = at[k] = (uint32_t)total;
+            total += size[k];
+        }
+        for (BatchView& B : bv)
+            for (uint32_t k = 0; k < kQueues; ++k) {
+                uint32_t& next = at[B.traversal * kQueues + k];
+                B.first[k] = next;
+                next += TileDeal{B.tiles_x, B.rows, B.rpl, sw, sh}.total(k);
+            }
     }
     if (total > 0xFFFFFFFFull) return fail(XD_ERR_INVALID_ARGUMENT, "%llu wave tiles in one batch", (unsigned long long)total);
-    T.qbeg[kClasses * kQueues] = (uint32_t)total;
-    T.tiles.clear();
-    T.tiles.reserve(total);
+    T.qbeg[kClasses * kQueues] = T.total_tiles = (uint32_t)total;
     for (auto& v : q) T.tiles.insert(T.tiles.end(), v.begin(), v.end());
     for (uint32_t c = 0; c < kClasses; ++c) cls.tiles[c] = T.qbeg[(c + 1) * kQueues] - T.qbeg[c * kQueues];
     cls.tiles[kClasses] = (uint32_t)total;
     T.cls = cls;
     return XD_OK;
+}
+
+// Writes the tile table on s: what the host dealt, or the device's deal.
+hipError_t write_tiles(const HostTables& T, uint32_t order, const BatchView* d_views, uint32_t* d_tiles, hipStream_t s) {
+    if (T.total_tiles == 0) return hipSuccess;
+    if (!T.tiles.empty())
+        return hipMemcpyAsync(d_tiles, T.tiles.data(), sizeof(uint32_t) * T.total_tiles, hipMemcpyHostToDevice, s);
+    hipLaunchKernelGGL(k_deal_tiles, dim3((T.most_tiles + 255) / 256, (uint32_t)T.views.size()), dim3(256), 0, s, d_views,
+                       square_width(order), square_height(order), d_tiles);
+    return hipGetLastError();
 }
 
 // Builds the current views' tables and uploads them into the batch's own
@@ -498,13 +580,16 @@ int upload_tables(xd_batch* b, BatchClasses* need) {
     int rc = build_tables(b->views.data(), n, b->tuning, T, b->keep_mixed);
     if (rc) return rc;
     b->total_rays = T.total_rays;
-    const uint32_t total = (uint32_t)T.tiles.size();
-    if ((rc = ensure_capacity(b, n, std::max<uint32_t>(total, 1)))) return rc;
+    if ((rc = ensure_capacity(b, n, std::max<uint32_t>(T.total_tiles, 1)))) return rc;
     hipError_t e;
-    if ((e = hipMemcpy(b->d_views, T.views.data(), sizeof(BatchView) * n, hipMemcpyHostToDevice)) != hipSuccess ||
-        (total && (e = hipMemcpy(b->d_tiles, T.tiles.data(), sizeof(uint32_t) * total, hipMemcpyHostToDevice)) != hipSuccess) ||
-        (e = hipMemcpy(b->d_qbeg, T.qbeg, sizeof(T.qbeg), hipMemcpyHostToDevice)) != hipSuccess)
+    hipStream_t s = b->ctx->stream;
+    if ((e = hipMemcpyAsync(b->d_views, T.views.data(), sizeof(BatchView) * n, hipMemcpyHostToDevice, s)) != hipSuccess ||
+        (e = hipMemcpyAsync(b->d_qbeg, T.qbeg, sizeof(T.qbeg), hipMemcpyHostToDevice, s)) != hipSuccess ||
+        (e = write_tiles(T, b->tuning.interleave, b->d_views, b->d_tiles, s)) != hipSuccess ||
+        (e = hipStreamSynchronize(s)) != hipSuccess) {
+        (void)hipStreamSynchronize(s);  // no copy may still read the host tables when they go
         return fail_hip(e, "batch tables");
+    }
     *need = T.cls;
     return XD_OK;
 }
@@ -842,7 +927,7 @@ int xd_batch_render_static(xd_context* ctx, const xd_view* views, uint32_t count
     if (rays) *rays = T.total_rays;
     if (ms) *ms = 0;
     if (count == 0) return XD_OK;
-    const uint32_t total = (uint32_t)T.tiles.size();
+    const uint32_t total = T.total_tiles;
     if (total > kStaticTiles)
         return fail(XD_ERR_INVALID_ARGUMENT, "%u wave tiles exceed the static limit of %u", total, kStaticTiles);
     const bool w8 = tun.waves_per_simd == 8;
@@ -859,7 +944,7 @@ int xd_batch_render_static(xd_context* ctx, const xd_view* views, uint32_t count
     hipStream_t s = ctx->stream;
     // launch_batch clears the counters with a kernel before the class kernels
     if ((e = hipMemcpyAsync(d_views, T.views.data(), sizeof(BatchView) * count, hipMemcpyHostToDevice, s)) != hipSuccess ||
-        (total && (e = hipMemcpyAsync(d_tiles, T.tiles.data(), sizeof(uint32_t) * total, hipMemcpyHostToDevice, s)) != hipSuccess) ||
+        (e = write_tiles(T, tun.interleave, d_views, d_tiles, s)) != hipSuccess ||
         (e = hipMemcpyAsync(d_qbeg, T.qbeg, sizeof(T.qbeg), hipMemcpyHostToDevice, s)) != hipSuccess ||
         (e = hipEventRecord(ctx->ev0, s)) != hipSuccess ||
         (e = launch_batch(d_views, d_tiles, d_qbeg, d_counters, pack_grabs(tun.tiles_per_grab, tun.rays_per_lane), cls,

@@ -9,19 +9,21 @@
 
 namespace xd {
 
+constexpr uint32_t kQueues = 8;                 // one tile range per XCD, per traversal class
+constexpr uint32_t kClasses = 5;                // one persistent kernel per traversal
+constexpr uint32_t kMaxBatchViews = 1u << 12;   // a tile entry is (view << 20 | tile)
+constexpr uint32_t kMaxTilesPerView = 1u << 20;
+
 // One output of a launch: its kernel parameters and wave-tile geometry.
 struct BatchView {
     RenderParams p;
     uint32_t traversal;
     uint32_t tw_shift;  // log2 of the tile width
     uint32_t tiles_x;
+    uint32_t rows;            // rows of wave tiles, in groups of rpl
+    uint32_t first[kQueues];  // where the device deals the tiles: its entries of each queue begin here
     uint32_t rpl;       // rays per lane: rows of wave tiles queued and grabbed together
 };
-
-constexpr uint32_t kQueues = 8;                 // one tile range per XCD, per traversal class
-constexpr uint32_t kClasses = 5;                // one persistent kernel per traversal
-constexpr uint32_t kMaxBatchViews = 1u << 12;   // a tile entry is (view << 20 | tile)
-constexpr uint32_t kMaxTilesPerView = 1u << 20;
 
 // Words between the counters of two ranges: a cache line each, so that grabs
 // from different ranges do not wait for one another (eight 1080p dda frames:
