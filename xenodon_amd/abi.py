@@ -559,7 +559,7 @@ class Frame:
         self.height = hgt
 
     def download(self):
-        out = np.zeros((self.height, self.width, 4), np.uint8)
+        out = np.empty((self.height, self.width, 4), np.uint8)
         check(lib().xd_frame_download(self.h, out.ctypes.data, 0))
         return out
 
@@ -592,10 +592,9 @@ def build_octree(grid, heuristic=HEURISTIC_CHAN_DIFF, chan_diff=0, std_dev=0.0, 
 
 
 def _take_nodes(out, st):
+    # the array is the library's buffer, released with the last view of it
     n = st.node_count
-    try:
-        buf = (ctypes.c_uint32 * (n * 10)).from_address(out.value)
-        nodes = np.frombuffer(buf, dtype=np.uint32).reshape(n, 10).copy()
-    finally:
-        lib().xd_free(out)
+    buf = (ctypes.c_uint32 * (n * 10)).from_address(out.value)
+    weakref.finalize(buf, lib().xd_free, ctypes.c_void_p(out.value))
+    nodes = np.frombuffer(buf, dtype=np.uint32).reshape(n, 10)
     return nodes, {f: getattr(st, f) for f, _ in BuildStats._fields_}

@@ -773,13 +773,16 @@ int xd_build_octree_device(xd_context* ctx, const xd_volume* grid, int heuristic
         }
         XD_TRY(hipGetLastError(), "octree build: ropes");
     }
-    uint32_t* host = static_cast<uint32_t*>(malloc((size_t)U * 40));
+    uint32_t* host = static_cast<uint32_t*>(alloc_large((uint64_t)U * 40));
     if (!host) {
         cleanup();
         return fail(XD_ERR_OUT_OF_MEMORY, "out of host memory for %u nodes", U);
     }
-    XD_TRY(hipMemcpyAsync(host, d_nodes, (size_t)U * 40, hipMemcpyDeviceToHost, s), "octree build: download");
-    XD_TRY(hipStreamSynchronize(s), "octree build: download");
+    if ((e = read_back(ctx, d_nodes, host, (uint64_t)U * 40, 1, (uint64_t)U * 40)) != hipSuccess) {
+        cleanup();
+        free(host);
+        return fail_hip(e, "octree build: download");
+    }
     cleanup();
 #undef XD_TRY
     stats->total_leaves = leaves;

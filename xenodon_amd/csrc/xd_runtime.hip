@@ -6,13 +6,18 @@
 //   HeadlessOutput::{synchronize, download}     -> xd_render's wait, xd_frame_download
 #include <hip/hip_runtime.h>
 
+#include <sys/mman.h>
+
 #include <algorithm>
+#include <atomic>
 #include <cstdarg>
 #include <cstdio>
+#include <cstdlib>
 #include <cstring>
 #include <memory>
 #include <new>
 #include <string>
+#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -163,6 +168,120 @@ uint64_t svo_footprint(uint64_t node_count, bool raw) {
     return node_count * 8 * sizeof(uint32_t) + node_count * sizeof(uint2) + kTableBytes;
 }
 
+namespace {
+
+hipError_t ensure_pin(xd_context* ctx) {
+    hipError_t e;
+    if (!ctx->pin && (e = hipHostMalloc(reinterpret_cast<void**>(&ctx->pin), kPinSlots * kPinSlot, hipHostMallocDefault)) !=
+                         hipSuccess) {
+        ctx->pin = nullptr;
+        return e;
+    }
+    for (hipEvent_t& ev : ctx->pin_ev)
+        if (!ev && (e = hipEventCreateWithFlags(&ev, hipEventDisableTiming)) != hipSuccess) {
+            ev = nullptr;
+            return e;
+        }
+    return hipSuccess;
+}
+
+}  // namespace
+
+void* alloc_large(uint64_t bytes) {
+    constexpr uint64_t huge = 2ull << 20;
+    if (bytes < 2 * huge) return malloc(bytes);
+    void* const p = aligned_alloc(huge, (bytes + huge - 1) / huge * huge);
+    if (p) (void)madvise(p, bytes, MADV_HUGEPAGE);
+    return p;
+}
+
+// The device writes a ring of pinned slots and several threads copy them out:
+// the host's pages are mostly fresh, and their faults, 5.8 ms for 33 MB on one
+// thread, cost ten times the transfer.  hipMemcpy2D to pageable memory took 0.7
+// ms whatever the size, and then the faults.  33 MB: 17.7 -> 1.8 ms; 113 KB: 1.0
+// -> 0.03.
+hipError_t read_back(xd_context* ctx, const void* src, void* dst, uint64_t row_bytes, uint64_t rows, uint64_t stride) {
+    hipStream_t s = ctx->stream;
+    hipError_t e = ensure_pin(ctx);
+    if (e != hipSuccess) {  // no pinned memory: the runtime's own copy
+        (void)hipGetLastError();
+        if ((e = hipStreamSynchronize(s)) != hipSuccess) return e;
+        return hipMemcpy2D(dst, stride, src, row_bytes, row_bytes, rows, hipMemcpyDeviceToHost);
+    }
+    if (stride == row_bytes) {
+        row_bytes *= rows;
+        rows = 1;
+    }
+    const uint8_t* const from = static_cast<const uint8_t*>(src);
+    uint8_t* const to = static_cast<uint8_t*>(dst);
+    // a slot takes whole rows, or a part of one
+    const bool split = row_bytes > kPinSlot;
+    const uint64_t per = split ? kPinSlot : kPinSlot / row_bytes * row_bytes;
+    const uint64_t per_row = split ? (row_bytes + per - 1) / per : 0;  // slots a row
+    const uint64_t n = split ? per_row * rows : (row_bytes * rows + per - 1) / per;
+    const auto begin = [&](uint64_t i) { return split ? i / per_row * row_bytes + i % per_row * per : i * per; };
+    const auto length = [&](uint64_t i) {
+        return split ? std::min(per, row_bytes - i % per_row * per) : std::min(per, row_bytes * rows - i * per);
+    };
+    const auto copy_out = [&](uint64_t i) {
+        const uint8_t* const p = ctx->pin + i % kPinSlots * kPinSlot;
+        if (split) {
+            memcpy(to + i / per_row * stride + i % per_row * per, p, length(i));
+        } else if (rows == 1) {
+            memcpy(to + i * per, p, length(i));
+        } else {
+            const uint64_t first = i * (per / row_bytes), count = length(i) / row_bytes;
+            for (uint64_t r = 0; r < count; ++r) memcpy(to + (first + r) * stride, p + r * row_bytes, row_bytes);
+        }
+    };
+    std::atomic<uint64_t> ready{0}, next{0};  // transfers done; the next one to copy out
+    std::atomic<uint64_t> emptied[kPinSlots];  // 1 + the last transfer copied out of each slot
+    for (auto& x : emptied) x.store(0);
+    std::atomic<bool> stop{false};
+    constexpr unsigned most = 8;
+    std::thread th[most];
+    unsigned threads = 0;
+    const unsigned want = n < 2 ? 0u : (unsigned)std::min<uint64_t>({n, most, std::max(1u, std::thread::hardware_concurrency())});
+    const auto worker = [&] {
+        for (uint64_t i; (i = next.fetch_add(1)) < n;) {
+            while (ready.load(std::memory_order_acquire) <= i) {
+                if (stop.load()) return;
+                std::this_thread::yield();
+            }
+            copy_out(i);
+            emptied[i % kPinSlots].store(i + 1, std::memory_order_release);
+        }
+    };
+    try {
+        for (; threads < want; ++threads) th[threads] = std::thread(worker);
+    } catch (const std::system_error&) {  // fewer threads, or none: then this one copies
+    }
+    constexpr uint64_t ahead = kPinSlots / 2;  // transfers queued before the oldest is waited for
+    for (uint64_t i = 0; i < n + ahead && e == hipSuccess; ++i) {
+        if (i < n) {
+            while (i >= kPinSlots && emptied[i % kPinSlots].load(std::memory_order_acquire) != i + 1 - kPinSlots)
+                std::this_thread::yield();
+            if ((e = hipMemcpyAsync(ctx->pin + i % kPinSlots * kPinSlot, from + begin(i), length(i), hipMemcpyDeviceToHost,
+                                    s)) != hipSuccess ||
+                (e = hipEventRecord(ctx->pin_ev[i % kPinSlots], s)) != hipSuccess)
+                break;
+        }
+        if (i < ahead || i - ahead >= n) continue;
+        const uint64_t k = i - ahead;
+        if ((e = hipEventSynchronize(ctx->pin_ev[k % kPinSlots])) != hipSuccess) break;
+        if (threads == 0) {
+            copy_out(k);
+            emptied[k % kPinSlots].store(k + 1, std::memory_order_release);
+        } else {
+            ready.store(k + 1, std::memory_order_release);
+        }
+    }
+    if (e != hipSuccess) stop.store(true);
+    for (unsigned t = 0; t < threads; ++t) th[t].join();
+    if (e != hipSuccess) (void)hipStreamSynchronize(s);  // nothing may still write the ring
+    return e;
+}
+
 int check_view(const xd_uniforms* u) {
     if (u->output_region.extent[0] == 0 || u->output_region.extent[1] == 0)
         return fail(XD_ERR_INVALID_ARGUMENT, "output region is empty");
@@ -284,6 +403,9 @@ int xd_close(xd_context* ctx) {
     std::vector<xd_frame*> frs(ctx->frames.begin(), ctx->frames.end());
     for (auto* f : frs) xd_frame_free(f);
     if (ctx->d_words) (void)hipFree(ctx->d_words);
+    for (hipEvent_t ev : ctx->pin_ev)
+        if (ev) (void)hipEventDestroy(ev);
+    if (ctx->pin) (void)hipHostFree(ctx->pin);
     if (ctx->ev0) (void)hipEventDestroy(ctx->ev0);
     if (ctx->ev1) (void)hipEventDestroy(ctx->ev1);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
@@ -672,10 +794,7 @@ int xd_frame_download(xd_frame* f, uint32_t* dst, uint64_t stride_px) {
     if (stride_px == 0) stride_px = f->w;
     if (stride_px < f->w) return fail(XD_ERR_INVALID_ARGUMENT, "stride below frame width");
     hipError_t e = hipSetDevice(f->ctx->device);
-    if (e == hipSuccess) e = hipStreamSynchronize(f->ctx->stream);
-    if (e == hipSuccess)
-        e = hipMemcpy2D(dst, stride_px * 4, f->d_pixels, (size_t)f->w * 4, (size_t)f->w * 4, f->h,
-                        hipMemcpyDeviceToHost);
+    if (e == hipSuccess) e = read_back(f->ctx, f->d_pixels, dst, (uint64_t)f->w * 4, f->h, stride_px * 4);
     if (e != hipSuccess) return fail_hip(e, "frame download");
     return XD_OK;
 }

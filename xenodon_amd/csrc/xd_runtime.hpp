@@ -9,6 +9,12 @@
 #include "xenodon.h"
 #include "xd_internal.hpp"
 
+namespace xd {
+// Slots and bytes a slot of a context's readback ring: 16 MiB in all.
+constexpr uint32_t kPinSlots = 16;
+constexpr uint64_t kPinSlot = 1ull << 20;
+}  // namespace xd
+
 struct xd_context {
     int device = 0;
     int tile_w = 8;  // per-wavefront tile width: 8 (8x8), 16 (16x4), 32 (32x2)
@@ -17,6 +23,9 @@ struct xd_context {
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     unsigned long long* d_words = nullptr;
+    // pinned ring that readbacks go through, made by the first of them (read_back)
+    uint8_t* pin = nullptr;
+    hipEvent_t pin_ev[xd::kPinSlots] = {};
     // live objects created on this context; xd_close frees what is left
     std::unordered_set<struct xd_volume*> volumes;
     std::unordered_set<struct xd_frame*> frames;
@@ -67,6 +76,12 @@ struct xd_frame {
 namespace xd {
 
 int fail(int code, const char* fmt, ...);
+// Copies `rows` rows of row_bytes, contiguous on the device, to host rows
+// `stride` bytes apart, behind the work queued on ctx's stream, and waits.
+hipError_t read_back(xd_context* ctx, const void* src, void* dst, uint64_t row_bytes, uint64_t rows, uint64_t stride);
+// malloc for a large buffer that will be written once: whole huge pages, where
+// the system gives them, so that the first writes fault 512 times less often.
+void* alloc_large(uint64_t bytes);
 int fail_hip(hipError_t e, const char* what);
 void clear_error();
 const char* traversal_name(int t);
