@@ -25,7 +25,7 @@
 //
 // The std-dev heuristic (Grid.cpp:139-214) splits when sqrt(S / n) > limit,
 // where S is an FP64 sum over the node's voxels taken in z, y, x order.  A
-// node of at most 16^3 voxels sums them in that order in one thread, which is
+// node of at most 4^3 voxels sums them in that order in one thread, which is
 // the reference's S exactly.  A larger node sums them in parallel in
 // double-double, which fixes S only to within the rounding error of a
 // sequential sum (|S - exact| <= gamma_{n-1} * exact, the terms being >= 0);
@@ -104,35 +104,70 @@ __device__ CellStats box_stats(const GridDev& g, uint32_t ox, uint32_t oy, uint3
     return s;
 }
 
-// Level of 4^3 cells, one thread per cell (nc cells per axis).
-__global__ void k_stats_base(GridDev g, uint32_t nc, CellStats* out) {
-    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const uint64_t total = (uint64_t)nc * nc * nc;
-    if (i >= total) return;
-    const uint32_t x = (uint32_t)(i % nc), y = (uint32_t)((i / nc) % nc), z = (uint32_t)(i / ((uint64_t)nc * nc));
-    out[i] = box_stats(g, x * 4, y * 4, z * 4, 4);
+// One level of the statistics pyramid: the cells that reach into the grid, nx by
+// ny by nz of them, x fastest.
+struct Cells {
+    CellStats* s;
+    uint32_t nx, ny, nz;
+    __device__ CellStats& at(uint32_t x, uint32_t y, uint32_t z) const { return s[((uint64_t)z * ny + y) * nx + x]; }
+};
+
+// Level of 4^3 cells, a cell's 16 rows in a quarter of a wave: a
+// lane takes its row's four texels with one load, and the quarter adds them up.
+// A thread a cell, with 64 loads, took 250 us for a 300x217x283 grid.
+__global__ __launch_bounds__(256) void k_stats_base(GridDev g, Cells out) {
+    const uint64_t t = (uint64_t)blockIdx.x * 256 + threadIdx.x, i = t >> 4;
+    const uint32_t r = (uint32_t)t & 15u;
+    const uint64_t cells = (uint64_t)out.nx * out.ny * out.nz;  // the bricks, in their order
+    uint32_t n = 0, sum[4] = {0, 0, 0, 0}, mn = 0xFFFFFFFFu, mx = 0;
+    if (i < cells) {
+        const uint32_t x = (uint32_t)(i % g.nbx), y = (uint32_t)((i / g.nbx) % g.nby), z = (uint32_t)(i / g.nbx / g.nby);
+        if (y * 4 + (r & 3u) < g.Y && z * 4 + (r >> 2) < g.Z) {
+            const uint4 v = *reinterpret_cast<const uint4*>(g.bricks + i * 64 + r * 4);
+            const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+            n = min(4u, g.X - x * 4);
+            for (uint32_t q = 0; q < n; ++q) {
+                for (int c = 0; c < 4; ++c) sum[c] += (w[q] >> (8 * c)) & 0xFFu;
+                mn = byte_min(mn, w[q]);
+                mx = byte_max(mx, w[q]);
+            }
+        }
+    }
+#pragma unroll
+    for (int d = 1; d < 16; d <<= 1) {
+        n += __shfl_xor(n, d, 64);
+        for (int c = 0; c < 4; ++c) sum[c] += __shfl_xor(sum[c], d, 64);
+        mn = byte_min(mn, __shfl_xor(mn, d, 64));
+        mx = byte_max(mx, __shfl_xor(mx, d, 64));
+    }
+    if (i < cells && r == 0) {
+        CellStats s{};
+        s.n = n;
+        for (int c = 0; c < 4; ++c) s.sum[c] = sum[c];
+        s.mn = mn;
+        s.mx = mx;
+        out.s[i] = s;
+    }
 }
 
-// Parent level from a child level of 2*nc cells per axis.
-__global__ void k_stats_merge(const CellStats* child, uint32_t nc, CellStats* out) {
+// Parent level from a child level.
+__global__ void k_stats_merge(Cells child, Cells out) {
     const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const uint64_t total = (uint64_t)nc * nc * nc;
-    if (i >= total) return;
-    const uint32_t x = (uint32_t)(i % nc), y = (uint32_t)((i / nc) % nc), z = (uint32_t)(i / ((uint64_t)nc * nc));
-    const uint64_t cn = 2ull * nc;
+    if (i >= (uint64_t)out.nx * out.ny * out.nz) return;
+    const uint32_t x = (uint32_t)(i % out.nx), y = (uint32_t)((i / out.nx) % out.ny), z = (uint32_t)(i / out.nx / out.ny);
     CellStats s{};
     s.mn = 0xFFFFFFFFu;
     s.mx = 0;
     for (int k = 0; k < 8; ++k) {
-        const uint64_t cx = 2ull * x + ((k >> 2) & 1), cy = 2ull * y + ((k >> 1) & 1), cz = 2ull * z + (k & 1);
-        const CellStats& c = child[(cz * cn + cy) * cn + cx];
-        if (!c.n) continue;
+        const uint32_t cx = 2 * x + ((k >> 2) & 1), cy = 2 * y + ((k >> 1) & 1), cz = 2 * z + (k & 1);
+        if (cx >= child.nx || cy >= child.ny || cz >= child.nz) continue;
+        const CellStats& c = child.at(cx, cy, cz);
         s.n += c.n;
         for (int q = 0; q < 4; ++q) s.sum[q] += c.sum[q];
         s.mn = byte_min(s.mn, c.mn);
         s.mx = byte_max(s.mx, c.mx);
     }
-    out[i] = s;
+    out.s[i] = s;
 }
 
 __device__ __forceinline__ void decode(uint64_t code, uint32_t level, uint32_t& x, uint32_t& y, uint32_t& z) {
@@ -185,11 +220,11 @@ __device__ __forceinline__ uint32_t sd_side(double s_lo, double s_hi, double nd,
 
 // Classifies the nodes of one level.  stats = that level's pyramid (cells of
 // extent >= 4), or nullptr to scan the grid (extent 2 and 1).  heuristic 1
-// (std-dev): big = this level's double-double sums (extent >= 32), and nodes
+// (std-dev): big = this level's double-double sums (extent >= 8), and nodes
 // whose split cannot be decided here are listed in amb (count in amb_n) and
 // left internal until the host decides.
 __global__ void k_classify(GridDev g, const uint64_t* codes, uint64_t count, uint32_t level, uint32_t extent,
-                           const CellStats* stats, uint32_t nc, uint32_t heuristic, uint32_t chan_diff, double sd_limit,
+                           Cells stats, uint32_t heuristic, uint32_t chan_diff, double sd_limit,
                            const double2* big, uint32_t* amb, uint32_t* amb_n, uint32_t* colour, uint32_t* internal) {
     const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= count) return;
@@ -198,8 +233,8 @@ __global__ void k_classify(GridDev g, const uint64_t* codes, uint64_t count, uin
     const uint64_t ox = (uint64_t)cx * extent, oy = (uint64_t)cy * extent, oz = (uint64_t)cz * extent;
     uint32_t col = 0, inner = 0;
     if (ox < g.X && oy < g.Y && oz < g.Z) {
-        const CellStats s = stats ? stats[((uint64_t)cz * nc + cy) * nc + cx]
-                                  : box_stats(g, (uint32_t)ox, (uint32_t)oy, (uint32_t)oz, extent);
+        const CellStats s = stats.s ? stats.at(cx, cy, cz)
+                                    : box_stats(g, (uint32_t)ox, (uint32_t)oy, (uint32_t)oz, extent);
         uint32_t diff = 0;
         for (int c = 0; c < 4; ++c) {
             col |= (uint32_t)(uint8_t)(s.sum[c] / s.n) << (8 * c);
@@ -238,36 +273,16 @@ __global__ void k_classify(GridDev g, const uint64_t* codes, uint64_t count, uin
 }
 
 // Double-double sum of the std-dev terms of node i's voxels (one block per
-// node; a level of nodes of extent >= 32).
+// node and part; a level of nodes of extent >= 8).
 __device__ __forceinline__ void two_sum(double a, double b, double& s, double& e) {
     s = a + b;
     const double bb = s - a;
     e = (a - (s - bb)) + (b - bb);
 }
 
-__global__ __launch_bounds__(256) void k_stddev_big(GridDev g, const uint64_t* codes, uint32_t level, uint32_t extent,
-                                                    const CellStats* stats, uint32_t nc, double2* out) {
-    const uint64_t i = blockIdx.x;
-    uint32_t cx, cy, cz;
-    decode(codes[i], level, cx, cy, cz);
-    const uint64_t ox = (uint64_t)cx * extent, oy = (uint64_t)cy * extent, oz = (uint64_t)cz * extent;
+// Sum of (hi, lo) pairs over a block of 256.
+__device__ __forceinline__ void block_sum_dd(double hi, double lo, double2* out) {
     __shared__ double hs[256], ls[256];
-    double hi = 0, lo = 0;
-    if (ox < g.X && oy < g.Y && oz < g.Z) {
-        const CellStats st = stats[((uint64_t)cz * nc + cy) * nc + cx];
-        double avg[4];
-        sd_avg(st, avg);
-        const uint64_t wx = min(ox + extent, (uint64_t)g.X) - ox, wy = min(oy + extent, (uint64_t)g.Y) - oy;
-        const uint64_t wz = min(oz + extent, (uint64_t)g.Z) - oz;
-        const uint64_t n = wx * wy * wz;
-        for (uint64_t k = threadIdx.x; k < n; k += blockDim.x) {
-            const uint64_t x = ox + k % wx, y = oy + (k / wx) % wy, z = oz + k / (wx * wy);
-            double s, e;
-            two_sum(hi, sd_term(g.texel((uint32_t)x, (uint32_t)y, (uint32_t)z), avg), s, e);
-            hi = s;
-            lo += e;
-        }
-    }
     hs[threadIdx.x] = hi;
     ls[threadIdx.x] = lo;
     __syncthreads();
@@ -280,12 +295,62 @@ __global__ __launch_bounds__(256) void k_stddev_big(GridDev g, const uint64_t* c
         }
         __syncthreads();
     }
-    if (threadIdx.x == 0) out[i] = make_double2(hs[0], ls[0]);
+    if (threadIdx.x == 0) *out = make_double2(hs[0], ls[0]);
+}
+
+// Part blockIdx.x of node blockIdx.y + first, a row of four texels a thread at a
+// time: rows part, part + parts, ... in blocks of 256.  The extent (8 or more)
+// is a power of two, so a row's place follows from its bits.  A block a node,
+// with divisions for every voxel, had left the upper levels on a few CUs: 4.7 ms
+// for a 128^3 grid, now 0.05.
+__global__ __launch_bounds__(256) void k_stddev_big(GridDev g, const uint64_t* codes, uint64_t first, uint32_t level,
+                                                    uint32_t extent, Cells stats, double2* out) {
+    const uint64_t i = first + blockIdx.y;
+    uint32_t cx, cy, cz;
+    decode(codes[i], level, cx, cy, cz);
+    const uint64_t ox = (uint64_t)cx * extent, oy = (uint64_t)cy * extent, oz = (uint64_t)cz * extent;
+    double hi = 0, lo = 0;
+    if (ox < g.X && oy < g.Y && oz < g.Z) {
+        double avg[4];
+        sd_avg(stats.at(cx, cy, cz), avg);
+        const uint32_t b = 29u - __builtin_clz(extent);  // log2 of the extent in bricks
+        const uint64_t rows = (uint64_t)extent * extent * extent / 4;
+        for (uint64_t k = (uint64_t)blockIdx.x * 256 + threadIdx.x; k < rows; k += (uint64_t)gridDim.x * 256) {
+            const uint32_t r = (uint32_t)k & 15u;
+            const uint64_t brick = k >> 4;
+            const uint32_t m = (1u << b) - 1u;
+            const uint64_t bx = (ox >> 2) + (brick & m), by = (oy >> 2) + (brick >> b & m), bz = (oz >> 2) + (brick >> (2 * b));
+            if (bx >= g.nbx || by * 4 + (r & 3u) >= g.Y || bz * 4 + (r >> 2) >= g.Z) continue;
+            const uint4 v = *reinterpret_cast<const uint4*>(g.bricks + ((bz * g.nby + by) * g.nbx + bx) * 64 + r * 4);
+            const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+            const uint32_t n = (uint32_t)min((uint64_t)4, g.X - bx * 4);
+            for (uint32_t q = 0; q < n; ++q) {
+                double s, e;
+                two_sum(hi, sd_term(w[q], avg), s, e);
+                hi = s;
+                lo += e;
+            }
+        }
+    }
+    block_sum_dd(hi, lo, out + i * gridDim.x + blockIdx.x);
+}
+
+// The parts of a node's sum, one block a node.
+__global__ __launch_bounds__(256) void k_stddev_join(const double2* parts, uint32_t count, double2* out) {
+    double hi = 0, lo = 0;
+    for (uint32_t k = threadIdx.x; k < count; k += 256) {
+        const double2 p = parts[(uint64_t)blockIdx.x * count + k];
+        double s, e;
+        two_sum(hi, p.x, s, e);
+        hi = s;
+        lo += e + p.y;
+    }
+    block_sum_dd(hi, lo, out + blockIdx.x);
 }
 
 // The reference's sequential S for the nodes k_classify could not decide.
 __global__ void k_stddev_exact(GridDev g, const uint64_t* codes, uint32_t level, uint32_t extent,
-                               const CellStats* stats, uint32_t nc, const uint32_t* amb, uint32_t n_amb, double* sums,
+                               Cells stats, const uint32_t* amb, uint32_t n_amb, double* sums,
                                double* counts) {
     const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= n_amb) return;
@@ -293,8 +358,8 @@ __global__ void k_stddev_exact(GridDev g, const uint64_t* codes, uint32_t level,
     uint32_t cx, cy, cz;
     decode(codes[i], level, cx, cy, cz);
     const uint64_t ox = (uint64_t)cx * extent, oy = (uint64_t)cy * extent, oz = (uint64_t)cz * extent;
-    const CellStats st = stats ? stats[((uint64_t)cz * nc + cy) * nc + cx]
-                               : box_stats(g, (uint32_t)ox, (uint32_t)oy, (uint32_t)oz, extent);
+    const CellStats st = stats.s ? stats.at(cx, cy, cz)
+                                 : box_stats(g, (uint32_t)ox, (uint32_t)oy, (uint32_t)oz, extent);
     double avg[4];
     sd_avg(st, avg);
     sums[j] = sd_sequential(g, ox, oy, oz, extent, avg);
@@ -352,18 +417,15 @@ __global__ void k_emit(uint64_t count, uint32_t level, uint32_t n_total, const u
     const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= count) return;
     const uint32_t f = n_total - 1u - (start[i] + size[i] - 1u);
-    uint32_t* w = nodes + (uint64_t)f * 10;
-    if (internal[i]) {
+    uint2* const w = reinterpret_cast<uint2*>(nodes + (uint64_t)f * 10);
+    uint32_t c[8] = {};
+    if (internal[i])
         for (uint32_t k = 0; k < 8; ++k) {
-            const uint64_t c = 8ull * rank[i] + k;
-            w[k] = n_total - 1u - (child_start[c] + child_size[c] - 1u);
+            const uint64_t at = 8ull * rank[i] + k;
+            c[k] = n_total - 1u - (child_start[at] + child_size[at] - 1u);
         }
-        w[9] = level;
-    } else {
-        for (uint32_t k = 0; k < 8; ++k) w[k] = 0;
-        w[9] = LEAF | level;
-    }
-    w[8] = colour[i];
+    for (uint32_t k = 0; k < 4; ++k) w[k] = make_uint2(c[2 * k], c[2 * k + 1]);
+    w[4] = make_uint2(colour[i], internal[i] ? level : LEAF | level);
 }
 
 // ---- DAG: equal nodes of one level, bottom-up ------------------------------
@@ -485,13 +547,17 @@ __global__ void k_ropes(const uint64_t* codes, uint64_t count, uint32_t level, u
     const uint64_t p[3] = {(uint64_t)cx * extent, (uint64_t)cy * extent, (uint64_t)cz * extent};
     uint32_t r[6];
     for (int a = 0; a < 3; ++a) {
+        // one neighbour along the axis is a sibling, the node that the walk to
+        // this level ends at: no walk for it
+        const uint64_t bit = 4u >> a, sib = i ^ bit;
+        const bool high = level != 0 && (i & bit) != 0;
+        const uint32_t sibling = level == 0 ? 0u : n_total - 1u - (start[sib] + size[sib] - 1u);
         uint64_t q[3] = {p[0], p[1], p[2]};
-        q[a] = p[a] + extent;
-        uint64_t f = find_node(nodes, side, q[0], q[1], q[2], level);
-        r[2 * a] = f == ~0ull ? 0u : (uint32_t)f;
-        q[a] = p[a] - extent;  // wraps below zero like size_t
-        f = find_node(nodes, side, q[0], q[1], q[2], level);
-        r[2 * a + 1] = f == ~0ull ? 0u : (uint32_t)f;
+        q[a] = high || level == 0 ? p[a] + extent : p[a] - extent;  // wraps below zero like size_t
+        const uint64_t f = find_node(nodes, side, q[0], q[1], q[2], level);
+        const uint32_t far = f == ~0ull ? 0u : (uint32_t)f;
+        r[2 * a] = high || level == 0 ? far : sibling;
+        r[2 * a + 1] = high ? sibling : level == 0 ? 0u : far;  // nothing is below a root
     }
     const uint32_t fi = n_total - 1u - (start[i] + size[i] - 1u);
     for (int k = 0; k < 6; ++k) nodes[(uint64_t)fi * 10 + k] = r[k];
@@ -536,16 +602,40 @@ int xd_build_octree_device(xd_context* ctx, const xd_volume* grid, int heuristic
     const GridDev g{grid->d_bricks, (uint32_t)grid->dims[0], (uint32_t)grid->dims[1], (uint32_t)grid->dims[2],
                     grid->nb[0], grid->nb[1], grid->nb[2]};
 
-    std::vector<void*> owned;
-    auto alloc = [&](void** p, size_t bytes) -> hipError_t {
-        hipError_t r = hipMalloc(p, std::max<size_t>(bytes, 16));
-        if (r == hipSuccess) owned.push_back(*p);
-        return r;
+    // One arena of a few blocks: an allocation and its release cost 70 us (0.4 ms
+    // from 128 MiB on, whatever the size), and a build makes 75 (rope) to 140
+    // (DAG) of them, more than its kernels took.  The first block is what a
+    // lossless tree of a body like a CT scan needs, 25 bytes a voxel.
+    std::vector<void*> blocks;
+    uint8_t* at = nullptr;
+    uint64_t left = 0, block_bytes = std::min<uint64_t>(
+        std::max<uint64_t>(32ull << 20, grid->dims[0] * grid->dims[1] * grid->dims[2] * 25), 4ull << 30);
+    auto alloc = [&](void** p, uint64_t bytes) -> hipError_t {
+        bytes = (std::max<uint64_t>(bytes, 16) + 255) / 256 * 256;
+        if (bytes > left) {
+            uint64_t want = std::max(bytes, block_bytes);
+            void* block = nullptr;
+            hipError_t r = hipMalloc(&block, want);
+            if (r == hipErrorOutOfMemory && want > bytes) {  // no room to spare
+                (void)hipGetLastError();
+                want = bytes;
+                r = hipMalloc(&block, want);
+            }
+            if (r != hipSuccess) return r;
+            blocks.push_back(block);
+            at = static_cast<uint8_t*>(block);
+            left = want;
+            block_bytes = std::max<uint64_t>(std::min<uint64_t>(block_bytes * 2, 1ull << 30), 64ull << 20);
+        }
+        *p = at;
+        at += bytes;
+        left -= bytes;
+        return hipSuccess;
     };
     auto cleanup = [&]() {
         (void)hipStreamSynchronize(s);
-        for (void* p : owned) (void)hipFree(p);
-        owned.clear();
+        for (void* p : blocks) (void)hipFree(p);
+        blocks.clear();
     };
 #define XD_TRY(expr, what)                      \
     do {                                        \
@@ -556,20 +646,28 @@ int xd_build_octree_device(xd_context* ctx, const xd_volume* grid, int heuristic
         }                                       \
     } while (0)
 
+    // counts read between levels land in pinned memory (words of the readback ring)
+    uint32_t* words = nullptr;
+    uint32_t unpinned[4];
+    if (pinned_words(ctx, &words) != hipSuccess) {
+        (void)hipGetLastError();
+        words = unpinned;
+    }
+
     // 1. statistics pyramid: levels B = D-2 (4^3 cells) up to 0
     const int B = (int)D - 2;
-    std::vector<CellStats*> pyr(std::max(B + 1, 0), nullptr);
-    if (B >= 0) {
-        const uint32_t ncb = 1u << B;
-        const uint64_t cells = (uint64_t)ncb * ncb * ncb;
-        XD_TRY(alloc((void**)&pyr[B], cells * sizeof(CellStats)), "octree build: statistics");
-        hipLaunchKernelGGL(k_stats_base, dim3(blocks_for(cells)), dim3(256), 0, s, g, ncb, pyr[B]);
-        for (int L = B - 1; L >= 0; --L) {
-            const uint32_t nc = 1u << L;
-            const uint64_t n = (uint64_t)nc * nc * nc;
-            XD_TRY(alloc((void**)&pyr[L], n * sizeof(CellStats)), "octree build: statistics");
-            hipLaunchKernelGGL(k_stats_merge, dim3(blocks_for(n)), dim3(256), 0, s, pyr[L + 1], nc, pyr[L]);
-        }
+    std::vector<Cells> pyr(std::max(B + 1, 0));
+    for (int L = B; L >= 0; --L) {
+        const uint64_t extent = side >> L;
+        Cells& c = pyr[L];
+        c = Cells{nullptr, (uint32_t)((g.X + extent - 1) / extent), (uint32_t)((g.Y + extent - 1) / extent),
+                  (uint32_t)((g.Z + extent - 1) / extent)};
+        const uint64_t n = (uint64_t)c.nx * c.ny * c.nz;
+        XD_TRY(alloc((void**)&c.s, n * sizeof(CellStats)), "octree build: statistics");
+        if (L == B)
+            hipLaunchKernelGGL(k_stats_base, dim3(blocks_for(n * 16)), dim3(256), 0, s, g, c);
+        else
+            hipLaunchKernelGGL(k_stats_merge, dim3(blocks_for(n)), dim3(256), 0, s, pyr[L + 1], c);
         XD_TRY(hipGetLastError(), "octree build: statistics");
     }
 
@@ -595,28 +693,35 @@ int xd_build_octree_device(xd_context* ctx, const xd_volume* grid, int heuristic
         XD_TRY(alloc((void**)&cur.rank, n * 4), "octree build: lists");
         const uint32_t extent = (uint32_t)std::min<uint64_t>(side >> L, 0xFFFFFFFFull);
         const bool from_pyr = (int)L <= B;
-        const uint32_t nc = 1u << std::min<uint32_t>(L, 31);
         double2* big = nullptr;
         uint32_t *amb = nullptr, *amb_n = nullptr;
         if (sd) {
             XD_TRY(alloc((void**)&amb, n * 4), "octree build: std-dev");
             XD_TRY(alloc((void**)&amb_n, 4), "octree build: std-dev");
             XD_TRY(hipMemsetAsync(amb_n, 0, 4, s), "octree build: std-dev");
-            if (from_pyr && extent >= 32) {
+            if (from_pyr && extent >= 8) {
+                // parts of at least 4096 voxels, enough of them to fill the device
+                const uint64_t voxels = (uint64_t)extent * extent * extent;
+                const uint32_t parts =
+                    (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(voxels / 4096, (4096 + n - 1) / n));
+                double2* part = nullptr;
                 XD_TRY(alloc((void**)&big, n * sizeof(double2)), "octree build: std-dev");
-                hipLaunchKernelGGL(k_stddev_big, dim3((unsigned)n), dim3(256), 0, s, g, cur.codes, L, extent, pyr[L],
-                                   nc, big);
+                XD_TRY(alloc((void**)&part, n * parts * sizeof(double2)), "octree build: std-dev");
+                for (uint64_t first = 0; first < n; first += 65535)  // the grid's second dimension
+                    hipLaunchKernelGGL(k_stddev_big, dim3(parts, (unsigned)std::min<uint64_t>(65535, n - first)), dim3(256),
+                                       0, s, g, cur.codes, first, L, extent, pyr[L], part);
+                hipLaunchKernelGGL(k_stddev_join, dim3((unsigned)n), dim3(256), 0, s, part, parts, big);
             }
         }
         hipLaunchKernelGGL(k_classify, dim3(blocks_for(n)), dim3(256), 0, s, g, cur.codes, n, L, extent,
-                           from_pyr ? pyr[L] : nullptr, nc, sd ? 1u : 0u, (uint32_t)chan_diff, std_dev, big, amb,
+                           from_pyr ? pyr[L] : Cells{}, sd ? 1u : 0u, (uint32_t)chan_diff, std_dev, big, amb,
                            amb_n, cur.colour, cur.internal);
         if (sd) {
             // nodes too close to the limit to decide on the device: the
             // reference's sequential S, and the converter's own comparison
-            uint32_t n_amb = 0;
-            XD_TRY(hipMemcpyAsync(&n_amb, amb_n, 4, hipMemcpyDeviceToHost, s), "octree build: std-dev");
+            XD_TRY(hipMemcpyAsync(&words[0], amb_n, 4, hipMemcpyDeviceToHost, s), "octree build: std-dev");
             XD_TRY(hipStreamSynchronize(s), "octree build: std-dev");
+            const uint32_t n_amb = words[0];
             if (n_amb) {
                 double *d_sums = nullptr, *d_counts = nullptr;
                 uint8_t* d_split = nullptr;
@@ -624,7 +729,7 @@ int xd_build_octree_device(xd_context* ctx, const xd_volume* grid, int heuristic
                 XD_TRY(alloc((void**)&d_counts, n_amb * 8ull), "octree build: std-dev");
                 XD_TRY(alloc((void**)&d_split, n_amb), "octree build: std-dev");
                 hipLaunchKernelGGL(k_stddev_exact, dim3(blocks_for(n_amb)), dim3(256), 0, s, g, cur.codes, L, extent,
-                                   from_pyr ? pyr[L] : nullptr, nc, amb, n_amb, d_sums, d_counts);
+                                   from_pyr ? pyr[L] : Cells{}, amb, n_amb, d_sums, d_counts);
                 std::vector<double> sums(n_amb), counts(n_amb);
                 std::vector<uint8_t> split(n_amb);
                 XD_TRY(hipMemcpyAsync(sums.data(), d_sums, n_amb * 8ull, hipMemcpyDeviceToHost, s), "octree build: std-dev");
@@ -647,12 +752,10 @@ int xd_build_octree_device(xd_context* ctx, const xd_volume* grid, int heuristic
         }
         XD_TRY(hipcub::DeviceScan::ExclusiveSum(tmp, tmp_bytes, cur.internal, cur.rank, (int)n, s),
                "octree build: scan");
-        uint32_t last_rank = 0, last_internal = 0;
-        XD_TRY(hipMemcpyAsync(&last_rank, cur.rank + n - 1, 4, hipMemcpyDeviceToHost, s), "octree build: scan");
-        XD_TRY(hipMemcpyAsync(&last_internal, cur.internal + n - 1, 4, hipMemcpyDeviceToHost, s),
-               "octree build: scan");
+        XD_TRY(hipMemcpyAsync(&words[0], cur.rank + n - 1, 4, hipMemcpyDeviceToHost, s), "octree build: scan");
+        XD_TRY(hipMemcpyAsync(&words[1], cur.internal + n - 1, 4, hipMemcpyDeviceToHost, s), "octree build: scan");
         XD_TRY(hipStreamSynchronize(s), "octree build: classify");
-        const uint64_t internals = (uint64_t)last_rank + last_internal;
+        const uint64_t internals = (uint64_t)words[0] + words[1];
         leaves += n - internals;
         if (internals == 0) break;
         Level next;
@@ -742,12 +845,12 @@ int xd_build_octree_device(xd_context* ctx, const xd_volume* grid, int heuristic
             tmp_bytes = need;
         }
         XD_TRY(hipcub::DeviceScan::ExclusiveSum(tmp, tmp_bytes, kept, ins, (int)N, s), "octree build: dag scan");
-        uint32_t last_ins = 0, last_kept = 0;
-        XD_TRY(hipMemcpyAsync(&last_ins, ins + N - 1, 4, hipMemcpyDeviceToHost, s), "octree build: dag scan");
-        XD_TRY(hipMemcpyAsync(&last_kept, kept + N - 1, 4, hipMemcpyDeviceToHost, s), "octree build: dag scan");
-        XD_TRY(hipMemcpyAsync(&unique_leaves, d_unique, 8, hipMemcpyDeviceToHost, s), "octree build: dag scan");
+        XD_TRY(hipMemcpyAsync(&words[0], ins + N - 1, 4, hipMemcpyDeviceToHost, s), "octree build: dag scan");
+        XD_TRY(hipMemcpyAsync(&words[1], kept + N - 1, 4, hipMemcpyDeviceToHost, s), "octree build: dag scan");
+        XD_TRY(hipMemcpyAsync(&words[2], d_unique, 8, hipMemcpyDeviceToHost, s), "octree build: dag scan");
         XD_TRY(hipStreamSynchronize(s), "octree build: dag scan");
-        U = last_ins + last_kept;
+        U = words[0] + words[1];
+        unique_leaves = words[2] | (unsigned long long)words[3] << 32;
     }
 
     // 4. nodes, then ropes

@@ -187,6 +187,12 @@ hipError_t ensure_pin(xd_context* ctx) {
 
 }  // namespace
 
+hipError_t pinned_words(xd_context* ctx, uint32_t** out) {
+    const hipError_t e = ensure_pin(ctx);
+    *out = reinterpret_cast<uint32_t*>(ctx->pin);
+    return e;
+}
+
 void* alloc_large(uint64_t bytes) {
     constexpr uint64_t huge = 2ull << 20;
     if (bytes < 2 * huge) return malloc(bytes);

@@ -79,6 +79,9 @@ int fail(int code, const char* fmt, ...);
 // Copies `rows` rows of row_bytes, contiguous on the device, to host rows
 // `stride` bytes apart, behind the work queued on ctx's stream, and waits.
 hipError_t read_back(xd_context* ctx, const void* src, void* dst, uint64_t row_bytes, uint64_t rows, uint64_t stride);
+// The first words of ctx's pinned ring (between readbacks), for counts that the
+// host waits for.
+hipError_t pinned_words(xd_context* ctx, uint32_t** out);
 // malloc for a large buffer that will be written once: whole huge pages, where
 // the system gives them, so that the first writes fault 512 times less often.
 void* alloc_large(uint64_t bytes);
