@@ -153,7 +153,7 @@ uint32_t macro_geometry(const uint64_t dims[3], uint32_t* shift, uint32_t mn[3])
 }
 
 // Device memory that a grid's upload goes through.
-constexpr uint64_t kGridStagingBytes = 256ull << 20;
+constexpr uint64_t kGridStagingBytes = 64ull << 20;
 
 uint64_t grid_footprint(const uint64_t dims[3]) {
     uint64_t nbricks = 1;
@@ -446,7 +446,8 @@ int xd_volume_from_grid(xd_context* ctx, const void* rgba8, uint64_t dim_x, uint
         return fail_hip(e, "grid allocation");
     }
     // several brick layers a copy: a copy of pageable memory costs about 0.1 ms
-    // beside its bytes.  Less where the device has no room for it.
+    // beside its bytes, and the release of 128 MB or more 0.3 ms.
+    // Less where the device has no room for it.
     uint64_t layers_at_once = kBrick;
     while (layers_at_once < dim_z && layers_at_once * 2 * layer_texels * sizeof(uint32_t) <= kGridStagingBytes)
         layers_at_once *= 2;
@@ -466,22 +467,24 @@ int xd_volume_from_grid(xd_context* ctx, const void* rgba8, uint64_t dim_x, uint
                            ctx->stream);
         if (e == hipSuccess)
             e = launch_bricks(staging, layers, (uint32_t)(z0 / kBrick), v->d_bricks, v->d_occ, dims32, v->nb, ctx->stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
         if (e != hipSuccess) {
+            (void)hipStreamSynchronize(ctx->stream);
             (void)hipFree(staging);
             xd_volume_free(v);
             return fail_hip(e, "grid upload");
         }
     }
-    (void)hipFree(staging);
     v->macro_words = macro_geometry(v->dims, &v->macro_shift, v->mn);
     if ((e = hipMalloc(&v->d_macro, (size_t)v->macro_words * 4)) != hipSuccess ||
         (e = launch_macro_mask(v->d_occ, v->nb, v->macro_shift, v->mn, v->d_macro, v->macro_words, ctx->stream)) !=
             hipSuccess ||
         (e = hipStreamSynchronize(ctx->stream)) != hipSuccess) {
+        (void)hipStreamSynchronize(ctx->stream);
+        (void)hipFree(staging);
         xd_volume_free(v);
         return fail_hip(e, "grid occupancy");
     }
+    (void)hipFree(staging);
     v->bytes += (uint64_t)v->macro_words * 4;
     ctx->volumes.insert(v);
     clear_error();
@@ -724,8 +727,8 @@ int xd_volume_free(xd_volume* v) {
     if (v->d_macro) (void)hipFree(v->d_macro);
     if (v->d_nodes) (void)hipFree(v->d_nodes);
     if (v->d_cw) (void)hipFree(v->d_cw);
-    if (v->d_meta) (void)hipFree(v->d_meta);
-    if (v->d_table) (void)hipFree(v->d_table);
+    if (v->d_meta && !v->one_block) (void)hipFree(v->d_meta);
+    if (v->d_table && !v->one_block) (void)hipFree(v->d_table);
     v->ctx->volumes.erase(v);
     delete v;
     return XD_OK;
