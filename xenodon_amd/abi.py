@@ -595,6 +595,7 @@ def _take_nodes(out, st):
     # the array is the library's buffer, released with the last view of it
     n = st.node_count
     buf = (ctypes.c_uint32 * (n * 10)).from_address(out.value)
-    weakref.finalize(buf, lib().xd_free, ctypes.c_void_p(out.value))
+    # (not at exit: an array that is still in use then goes with the process)
+    weakref.finalize(buf, lib().xd_free, ctypes.c_void_p(out.value)).atexit = False
     nodes = np.frombuffer(buf, dtype=np.uint32).reshape(n, 10)
     return nodes, {f: getattr(st, f) for f, _ in BuildStats._fields_}
