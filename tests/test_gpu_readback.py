@@ -36,3 +36,22 @@ def test_download_sizes_and_strides(W, Hh, pad):
             part, _ = ctx.render_image(vol, abi.DDA, cam, abi.make_uniforms(
                 w, h, [8] * 3, emission=1.5, out_offset=(x0, y0), disp_extent=(W, Hh)))
             assert np.array_equal(img[y0:y0 + h, x0:x0 + w], part)
+
+
+def test_download_waits_for_the_null_stream():
+    """A program that works on a frame's device memory on the null stream gets what that work wrote."""
+    hip = abi.lib()  # finds the HIP runtime's functions as well
+    hip.hipMalloc.argtypes = [ctypes.POINTER(ctypes.c_void_p), ctypes.c_size_t]
+    hip.hipMemsetAsync.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_size_t, ctypes.c_void_p]
+    hip.hipFree.argtypes = [ctypes.c_void_p]
+    size = 4 << 30
+    with abi.Context(0) as ctx:
+        fr = ctx.frame(640, 360)
+        buf = ctypes.c_void_p()
+        assert hip.hipMalloc(ctypes.byref(buf), size) == 0
+        for value in (3, 200):
+            for _ in range(8):  # some milliseconds
+                assert hip.hipMemsetAsync(buf, value, size, None) == 0
+            assert hip.hipMemsetAsync(fr.device_ptr(), value, 640 * 360 * 4, None) == 0
+            assert (fr.download() == value).all()
+        hip.hipFree(buf)

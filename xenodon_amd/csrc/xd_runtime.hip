@@ -803,6 +803,9 @@ int xd_frame_download(xd_frame* f, uint32_t* dst, uint64_t stride_px) {
     if (stride_px == 0) stride_px = f->w;
     if (stride_px < f->w) return fail(XD_ERR_INVALID_ARGUMENT, "stride below frame width");
     hipError_t e = hipSetDevice(f->ctx->device);
+    // the frame's device memory is the program's too (xd_frame_device_ptr): what it
+    // has queued on the null stream comes first, as for a hipMemcpy
+    if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
     if (e == hipSuccess) e = read_back(f->ctx, f->d_pixels, dst, (uint64_t)f->w * 4, f->h, stride_px * 4);
     if (e != hipSuccess) return fail_hip(e, "frame download");
     return XD_OK;
