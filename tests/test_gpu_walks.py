@@ -1,0 +1,94 @@
+"""The octree walks that take a short cut (esvo from cell to cell) against the
+general walk on the raw node words: trees at the edges of the short cut's range
+(1 level; the start table's 8 levels and one around them; the most levels and
+one more) and cameras that it must pass on or that meet cell borders exactly."""
+import numpy as np
+import pytest
+
+from tests.test_gpu_parity import _chain_tree
+from xenodon_amd import abi
+
+pytestmark = pytest.mark.gpu
+
+TARGET = (0.3712345, 0.6123457, 0.5317891)
+RAW = 1  # octree_layout: the node words as they are, which the general walk reads
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    if abi.device_count() < 1:
+        pytest.fail("no HIP device visible: GPU tests need an MI355X")
+    with abi.Context(0) as c:
+        yield c
+
+
+def _camera(eye, fwd, up=(0.0, 1.0, 0.0)):
+    f = np.array(fwd, float) / np.linalg.norm(fwd)
+    r = np.cross(up, f)
+    r /= np.linalg.norm(r)
+    return abi.make_camera(f, np.cross(f, r), eye)
+
+
+CAMERAS = {
+    "towards": lambda: _camera((-0.4, 1.1, -0.7), np.array(TARGET) - (-0.4, 1.1, -0.7)),
+    "back": lambda: _camera((1.3, 0.2, 1.6), np.array(TARGET) - (1.3, 0.2, 1.6)),
+    "inside": lambda: _camera(np.array(TARGET) + (2e-3, -1e-3, 3e-3), (-2.0, 1.0, -3.0)),
+    "axis": lambda: _camera((0.5, 0.5, -1.0), (0.0, 0.0, 1.0)),
+    "axis_inside": lambda: _camera((0.375, 0.625, 0.5), (-1.0, 0.0, 0.0)),
+    "diagonal": lambda: _camera((-0.5, 0.5, -0.5), (1.0, 0.0, 1.0)),
+    "corner": lambda: _camera((0.0, 0.0, 0.0), (1.0, 1.0, 1.0)),
+    "face": lambda: _camera((1.0, 0.25, 0.75), (0.0, 1.0, 1e-6)),
+    "away": lambda: _camera((-0.4, 1.1, -0.7), (-1.0, 0.2, -1.0)),
+    "far": lambda: _camera((3e4, 2e4, -1e4), np.array((0.5, 0.5, 0.5)) - (3e4, 2e4, -1e4)),
+}
+
+
+def _pair(ctx, nodes, side, t, cam, W=97, H=61):
+    uni = abi.make_uniforms(W, H, [side] * 3, emission=1.5)
+    images = []
+    for layout in (0, RAW):
+        ctx.set_option("octree_layout", layout)
+        try:
+            vol = ctx.svo_volume(nodes, side)
+        finally:
+            ctx.set_option("octree_layout", 0)
+        images.append(ctx.render_image(vol, t, cam, uni)[0])
+        vol.free()
+    return images
+
+
+@pytest.mark.parametrize("depth", [1, 2, 7, 8, 9, 10, 14, 15])
+@pytest.mark.parametrize("t", [abi.ESVO])
+def test_chain_trees(ctx, t, depth):
+    nodes = _chain_tree(depth, TARGET, seed=depth)
+    lit = 0
+    for name, cam in CAMERAS.items():
+        got, want = _pair(ctx, nodes, 1 << depth, t, cam())
+        assert np.array_equal(got, want), (name, int((got != want).any(-1).sum()))
+        lit += int(want[..., :3].any())
+    assert lit >= 6
+
+
+@pytest.mark.parametrize("bad", [float("nan"), float("inf"), 1e30])
+@pytest.mark.parametrize("axis", [0, 2])
+@pytest.mark.parametrize("t", [abi.ESVO])
+def test_cameras_out_of_range(ctx, t, axis, bad):
+    nodes = _chain_tree(9, TARGET, seed=3)
+    eye = [0.4, 0.6, -0.8]
+    eye[axis] = bad
+    got, want = _pair(ctx, nodes, 512, t, _camera(eye, (0.1, 0.05, 1.0)), 33, 17)
+    assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("tree", [abi.TREE_DAG, abi.TREE_SPARSE])
+@pytest.mark.parametrize("t", [abi.ESVO])
+def test_built_trees(ctx, t, tree):
+    """Every kind of leaf; the DAG has no records."""
+    rng = np.random.default_rng(8)
+    grid = rng.integers(0, 256, (24, 24, 24, 4), dtype=np.uint8)
+    grid[rng.random((24, 24, 24)) < 0.6] = 0
+    grid = np.kron(grid, np.ones((2, 2, 2, 1), np.uint8))
+    nodes, st = abi.build_octree(grid, tree=tree)
+    for name, cam in CAMERAS.items():
+        got, want = _pair(ctx, nodes, st["side"], t, cam())
+        assert np.array_equal(got, want), name

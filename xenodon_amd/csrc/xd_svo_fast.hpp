@@ -147,6 +147,70 @@ __device__ __forceinline__ uint32_t fast_find(const FastSvo& s, f3 pos, f3& base
     }
 }
 
+// The head of an internal node's record (RenderParams::rec).
+struct NodeRec {
+    uint32_t inner;  // first internal child
+    uint32_t masks;  // bits 0..7: internal children, 8..15: leaves with colour
+};
+
+typedef const __attribute__((address_space(1))) uint32_t* GlobalWords;
+
+__device__ __forceinline__ GlobalWords rec_words(const uint4* rec, uint32_t node) {
+    return (GlobalWords)rec + (uint64_t)node * kRecWords;
+}
+__device__ __forceinline__ NodeRec load_rec(GlobalWords w) {
+    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+    const u32x2 v = *(const __attribute__((address_space(1))) u32x2*)w;
+    return NodeRec{v.x, v.y};
+}
+
+// Computes v here: a sum that the compiler moves down past the load of its next
+// term makes the loop wait for that load in the same trip (199x143 frames of a
+// 128^3 volume by svo-naive: 0.120 -> 0.104 ms).
+__device__ __forceinline__ void pin(f3& v) { asm volatile("" : "+v"(v.x), "+v"(v.y), "+v"(v.z)); }
+
+// The leaf at the position with the bits bx, by, bz, from its cell's table entry:
+// its level, and its colour or null for none.  On records a node says of each
+// child whether it is a leaf and whether all of its own children are, so the leaf
+// is known one load earlier than by child words, and its colour is beside the
+// masks: 1080p frames of a 10-level tree (700x490x700 voxels) by svo-naive 1.38 /
+// 1.19 / 0.99 -> 1.05 / 0.87 / 0.86 ms.  One address for a leaf of either kind,
+// selected, cost 6 % on a 9-level tree.
+__device__ __forceinline__ uint32_t table_leaf(const FastSvo& s, const uint4* __restrict__ rec, uint2 e, uint32_t bx,
+                                               uint32_t by, uint32_t bz, const uint32_t*& colour) {
+    const auto octant = [&](uint32_t level) {
+        const uint32_t d = 22u - min(level, 22u);
+        return (bx >> d & 1u) << 2 | (by >> d & 1u) << 1 | (bz >> d & 1u);
+    };
+    const auto colour_in = [&](uint32_t node, uint32_t k) {  // of leaf k; 0 for an empty one
+        return reinterpret_cast<const uint32_t*>(rec) + (uint64_t)node * kRecWords + 4u + k;
+    };
+    uint32_t word = e.x, level = e.y & kTableLevelMask;
+    if (e.y & kTableLowNode) {
+        colour = colour_in(word & s.index_mask, octant(kTableLevel));
+        return kTableLevel + 1;
+    }
+    if (__builtin_expect(!(word & kTagLeaf), 0)) {
+        if (rec) {
+            for (;; ++level) {
+                const NodeRec r = load_rec(rec_words(rec, word & s.index_mask));
+                const uint32_t bit = 1u << octant(level);
+                if (!(r.masks & bit)) break;
+                word = r.inner + __popc(r.masks & (bit - 1u) & 0xFFu);
+                if (r.masks & (bit << 16)) {
+                    ++level;
+                    break;
+                }
+            }
+            colour = colour_in(word & s.index_mask, octant(level));
+            return level + 1;
+        }
+        for (; !(word & kTagLeaf) && level <= kMaxLevels; ++level) word = cw_at(s, word & s.index_mask, octant(level));
+    }
+    colour = empty_leaf(s, word) ? nullptr : s.meta + (word & s.index_mask);
+    return level;
+}
+
 // svo_naive.comp:29-71.  A step's position depends on the box of the leaf before
 // it, so a ray is one chain of loads; what is not on it is kept off it:
 //  * the start table says where a cell's node has only leaves for children.
@@ -187,21 +251,9 @@ __device__ __forceinline__ f3 fast_naive(const FastSvo& s, const uint4* __restri
             cell = at;
         }
         total = add(total, muls(unorm_rgb(pend_col), pend_w));  // +0 the first time
-        uint32_t word = e.x, level = e.y & kTableLevelMask;
-        const uint32_t* colour = s.meta;  // of the leaf, or null for none
-        if (e.y & kTableLowNode) {
-            const uint32_t k = (bx >> (sh - 1) & 1u) << 2 | (by >> (sh - 1) & 1u) << 1 | (bz >> (sh - 1) & 1u);
-            colour = reinterpret_cast<const uint32_t*>(rec) + (uint64_t)(word & s.index_mask) * kRecWords + 4u + k;
-            ++level;
-        } else {
-            while (!(word & kTagLeaf) && level <= kMaxLevels) {
-                const uint32_t d = 22u - min(level, 22u);
-                const uint32_t k = (bx >> d & 1u) << 2 | (by >> d & 1u) << 1 | (bz >> d & 1u);
-                word = cw_at(s, word & s.index_mask, k);
-                ++level;
-            }
-            colour = empty_leaf(s, word) ? nullptr : s.meta + (word & s.index_mask);
-        }
+        pin(total);
+        const uint32_t* colour;
+        const uint32_t level = table_leaf(s, rec, e, bx, by, bz, colour);
         // 1 + the leaf's corner is its leading bits after the point
         const uint32_t keep = ~0u << (23u - level);
         const f3 offset = mk(u2f(0x3F800000u | (bx & keep)) - 1.0f, u2f(0x3F800000u | (by & keep)) - 1.0f,
@@ -429,23 +481,6 @@ __device__ __forceinline__ f3 fast_df(const FastSvo& s, uint64_t cap, uint32_t s
     return total;
 }
 
-// The head of an internal node's record (RenderParams::rec).
-struct NodeRec {
-    uint32_t inner;  // first internal child
-    uint32_t masks;  // bits 0..7: internal children, 8..15: leaves with colour
-};
-
-typedef const __attribute__((address_space(1))) uint32_t* GlobalWords;
-
-__device__ __forceinline__ GlobalWords rec_words(const uint4* rec, uint32_t node) {
-    return (GlobalWords)rec + (uint64_t)node * kRecWords;
-}
-__device__ __forceinline__ NodeRec load_rec(GlobalWords w) {
-    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-    const u32x2 v = *(const __attribute__((address_space(1))) u32x2*)w;
-    return NodeRec{v.x, v.y};
-}
-
 // The walk of fast_df<true> on records.  It is bound by the instructions it
 // issues, half of the lanes busy, so it is built to need fewer trips:
 //  * empty leaves, which add exactly +0, leave the hit mask at once;
@@ -626,7 +661,7 @@ __device__ __forceinline__ f3 fast_rope(const FastSvo& s, uint64_t cap, f3 ro, f
     return total;
 }
 
-// esvo.comp:30-136
+// esvo.comp:30-136, for the trees and rays that fast_esvo_cells does not take.
 __device__ __forceinline__ f3 fast_esvo(const FastSvo& s, uint64_t cap, uint32_t slots, f3 ro, f3 rd,
                                         uint32_t* stk_parent, float* stk_tmax) {
     EsvoRay r = esvo_setup(ro, rd);
@@ -690,74 +725,117 @@ __device__ __forceinline__ f3 fast_esvo(const FastSvo& s, uint64_t cap, uint32_t
     return add(total, muls(unorm_rgb(pend_col), pend_w));
 }
 
-// The walk of fast_esvo on records: the parent's masks stay in registers, so a
-// step to a sibling needs no load but a leaf's colour, which is next to them in
-// memory, and an empty leaf is a clear bit.  1.28 / 1.28 / 3.75 -> 1.15 / 1.15 /
-// 3.58 ms on the frames above.
-__device__ __forceinline__ f3 fast_esvo_rec(const uint4* __restrict__ rec, uint32_t n, uint64_t cap, uint32_t slots,
-                                            f3 ro, f3 rd, uint32_t* stk_parent, float* stk_tmax) {
-    EsvoRay r = esvo_setup(ro, rd);
-    float t_min = r.t_min, t_max = r.t_max, h = r.h;
-    f3 pos = r.pos;
-    uint32_t idx = r.idx, parent = 0, scale = 22;
-    float scale_exp2 = 0.5f;
+// The walk of fast_esvo from cell to cell, for trees of 1 to kEsvoCellLevels
+// levels and rays that esvo_cell_ray accepts.
+//
+// The shader descends, steps and pops a level a trip; a wave's lanes do these in
+// turn, each trip costing what all of them cost.  Here a trip is one leaf, found
+// with one load of the start table, and there is no stack.  The terms, their order
+// and every float that enters a comparison or a sum are the shader's:
+//  * positions are 23-bit numbers, 1 + n * 2^-23 on the mirrored axes.  A descent's
+//    choices along an axis, t_center > t_min at each level, depend on that axis
+//    alone, and planes far from the ray's position at t_min fall as their distance
+//    says.  One plane can be near: the multiple m of the tree's finest cell that is
+//    nearest to (t_min + t_bias) * -|rd|.  Its comparison is made, as the shader
+//    makes it; the bits below are then 0...0 or 1...1.  (Positions are off by less
+//    than 2^-18 here, half of a finest cell is at least 2^-15.)  The descent starts
+//    in the cell that the step or pop leads to, so the result is clamped to that.
+//  * t_max is the least of the root's and the exits of the nodes entered, and an
+//    exit never lies behind its parent's: min(t_max of the root, the leaf's exit).
+//  * a node that t_min has passed already (t_center and its plane's t round apart)
+//    is skipped whole, so a skipped leaf looks for the outermost such node.
+// Plain 1080p frames of the 9-level tree above 1.06 / 1.12 / 3.50 -> 0.65 / 0.69 /
+// 2.08 ms, the three batched 4.98 -> 3.15; 10 levels 1.67 / 1.33 / 1.50 -> 1.02
+// / 0.82 / 1.09; a DAG without records 1.47 / 1.87 / 2.49 -> 0.86 / 1.08 / 1.51; a
+// 199x143 frame of a 128^3 volume 0.178 -> 0.113.
+constexpr uint32_t kEsvoCellLevels = 14;
+
+__device__ __forceinline__ bool esvo_cell_ray(f3 ro, f3 rd, const EsvoRay& r) {
+    const f3 d = mk(ro.x - 1.5f, ro.y - 1.5f, ro.z - 1.5f);
+    return r.t_min <= r.t_max && fabs_(d.x) <= 3.5f && fabs_(d.y) <= 3.5f && fabs_(d.z) <= 3.5f &&
+           fabs_(rd.x) <= 2.0f && fabs_(rd.y) <= 2.0f && fabs_(rd.z) <= 2.0f;
+}
+
+__device__ __forceinline__ float esvo_plane(int32_t n, float t_coeff, float t_bias) {
+    return u2f(0x3F800000u | (uint32_t)n) * t_coeff - t_bias;
+}
+
+// The cell along one axis at t_min, within the region of low bits `rest` around n.
+struct EsvoSnap {
+    float add;      // rounds a position to a multiple of the finest cell
+    uint32_t shift, base;
+};
+__device__ __forceinline__ int32_t esvo_cell(const EsvoSnap& q, float t_min, float neg_rd, float t_coeff, float t_bias,
+                                             int32_t n, int32_t rest) {
+    const float p = (t_min + t_bias) * neg_rd;
+    const int32_t m = (int32_t)((f2u(p + q.add) << q.shift) + q.base);
+    const int32_t half = m & -m;  // of the node that plane m divides
+    const float t_center = __builtin_fmaf((float)half, t_coeff * 0x1p-23f, esvo_plane(m - half, t_coeff, t_bias));
+    return max(n & ~rest, min(n | rest, t_center > t_min ? m : m - 1));
+}
+
+__device__ __forceinline__ f3 fast_esvo_cells(const FastSvo& s, const uint4* __restrict__ rec, uint32_t depth,
+                                              uint64_t cap, f3 rd, const EsvoRay& r) {
+    const uint32_t levels = max(depth, kTableLevel);
+    EsvoSnap q;
+    q.shift = 23u - levels;
+    q.add = __builtin_ldexpf(1.5f, (int)q.shift);  // its last place is 2^-levels
+    q.base = 0u - (f2u(q.add) << q.shift) - (1u << 23);
+    const f3 nd = mk(-fabs_(rd.x), -fabs_(rd.y), -fabs_(rd.z));
+    const uint32_t fx = (r.octant_mask & 4u) ? 0x7FFFFFu : 0u, fy = (r.octant_mask & 2u) ? 0x7FFFFFu : 0u,
+                   fz = (r.octant_mask & 1u) ? 0x7FFFFFu : 0u;
+    // the first cell: the root's child that esvo_setup chose
+    int32_t nx = (r.idx & 4u) ? 1 << 22 : 0, ny = (r.idx & 2u) ? 1 << 22 : 0, nz = (r.idx & 1u) ? 1 << 22 : 0;
+    int32_t rest = (1 << 22) - 1;
+    float t_min = r.t_min;
     f3 total = splat(0.0f);
-    uint32_t pend_col = 0;
+    uint32_t pend_col = 0;  // the last leaf's term, added at the next step
     float pend_w = 0.0f;
-    GlobalWords w = rec_words(rec, 0);
-    NodeRec nr = load_rec(w);
     const uint32_t cap32 = cap32_of(cap);
     uint32_t it = 0;
-    while (scale < 23u) {
-        if (++it > cap32) break;
-        f3 t_corner = sub(mul(pos, r.t_coeff), r.t_bias);
+    while (++it <= cap32) {
+        const int32_t cx = esvo_cell(q, t_min, nd.x, r.t_coeff.x, r.t_bias.x, nx, rest);
+        const int32_t cy = esvo_cell(q, t_min, nd.y, r.t_coeff.y, r.t_bias.y, ny, rest);
+        const int32_t cz = esvo_cell(q, t_min, nd.z, r.t_coeff.z, r.t_bias.z, nz, rest);
+        const uint32_t bx = (uint32_t)cx ^ fx, by = (uint32_t)cy ^ fy, bz = (uint32_t)cz ^ fz;
+        constexpr uint32_t sh = 23u - kTableLevel;
+        const uint2 e = s.table[table_cell(bx >> sh, by >> sh, bz >> sh)];
+        total = add(total, muls(unorm_rgb(pend_col), pend_w));  // +0 the first time
+        pin(total);
+        const uint32_t* colour;
+        const uint32_t level = table_leaf(s, rec, e, bx, by, bz, colour);
+        int32_t size = 1 << (23u - level);
+        int32_t lx = cx & -size, ly = cy & -size, lz = cz & -size;
+        f3 t_corner = mk(esvo_plane(lx, r.t_coeff.x, r.t_bias.x), esvo_plane(ly, r.t_coeff.y, r.t_bias.y),
+                         esvo_plane(lz, r.t_coeff.z, r.t_bias.z));
         float tc_max = min_elem(t_corner);
-        if (t_min <= t_max) {
-            float tv_max = gmin(t_max, tc_max);
-            if (t_min <= tv_max) {
-                const uint32_t ci = idx ^ r.octant_mask, bit = 1u << ci;
-                if (nr.masks & (bit << 8)) {
-                    const uint32_t col = w[4 + ci];
-                    total = add(total, muls(unorm_rgb(pend_col), pend_w));  // +0 the first time
-                    pend_col = col;
-                    pend_w = tv_max - t_min;
-                } else if (nr.masks & bit) {
-                    if (tc_max < h) {
-                        uint32_t slot = 22u - scale;
-                        if (slot < slots) {
-                            stk_parent[slot * kWaveLanes] = parent;
-                            stk_tmax[slot * kWaveLanes] = t_max;
-                        }
-                    }
-                    h = tc_max;
-                    parent = nr.inner + __popc(nr.masks & (bit - 1u) & 0xFFu);
-                    w = rec_words(rec, parent);
-                    nr = load_rec(w);
-                    --scale;
-                    scale_exp2 = scale_exp2 * 0.5f;
-                    f3 t_center = add(smul(scale_exp2, r.t_coeff), t_corner);
-                    bool ax = t_center.x > t_min, ay = t_center.y > t_min, az = t_center.z > t_min;
-                    idx = cxor(0u, ax, ay, az);
-                    pos = add(pos, mk(ax ? scale_exp2 : 0.0f, ay ? scale_exp2 : 0.0f, az ? scale_exp2 : 0.0f));
-                    t_max = tv_max;
-                    continue;
-                }
+        const float tv_max = gmin(r.t_max, tc_max);
+        pend_col = 0;
+        if (t_min <= tv_max) {
+            if (colour) pend_col = *colour;
+            pend_w = tv_max - t_min;
+        } else {
+            for (int32_t outer = rest + 1; outer > size; outer >>= 1) {
+                const f3 tc = mk(esvo_plane(cx & -outer, r.t_coeff.x, r.t_bias.x),
+                                 esvo_plane(cy & -outer, r.t_coeff.y, r.t_bias.y),
+                                 esvo_plane(cz & -outer, r.t_coeff.z, r.t_bias.z));
+                if (t_min <= gmin(r.t_max, min_elem(tc))) continue;
+                size = outer;
+                lx = cx & -size;
+                ly = cy & -size;
+                lz = cz & -size;
+                t_corner = tc;
+                tc_max = min_elem(tc);
+                break;
             }
         }
-        bool ax = t_corner.x <= tc_max, ay = t_corner.y <= tc_max, az = t_corner.z <= tc_max;
-        uint32_t step_mask = cxor(0u, ax, ay, az);
-        pos = sub(pos, mk(ax ? scale_exp2 : 0.0f, ay ? scale_exp2 : 0.0f, az ? scale_exp2 : 0.0f));
+        nx = lx - (t_corner.x <= tc_max ? size : 0);
+        ny = ly - (t_corner.y <= tc_max ? size : 0);
+        nz = lz - (t_corner.z <= tc_max ? size : 0);
+        if ((nx | ny | nz) < 0) break;
+        // the highest bit that changed is the size of the cell that the step leads to
+        rest = (int32_t)(0x7FFFFFFFu >> __builtin_clz((uint32_t)((lx ^ nx) | (ly ^ ny) | (lz ^ nz))));
         t_min = tc_max;
-        idx ^= step_mask;
-        if ((idx & step_mask) != 0) {
-            if (!esvo_pop(pos, scale_exp2, scale, idx, ax, ay, az)) break;
-            uint32_t slot = 22u - scale;
-            parent = slot < slots ? min(stk_parent[slot * kWaveLanes], n - 1u) : 0u;
-            t_max = slot < slots ? stk_tmax[slot * kWaveLanes] : 0.0f;
-            w = rec_words(rec, parent);
-            nr = load_rec(w);
-            h = 0.0f;
-        }
     }
     return add(total, muls(unorm_rgb(pend_col), pend_w));
 }

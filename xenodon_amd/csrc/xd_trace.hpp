@@ -274,17 +274,19 @@ __device__ __forceinline__ f3 svo_pixel(const RenderParams& p, f3 rd, uint32_t* 
     const FastSvo fs = make_fast_svo(p.cw, p.meta, p.root_tag, lds_top, n_top, p.node_count, p.depth_exact, p.table, p.rope_depth,
                       p.index_mask, p.empty_tag, p.empty_start, p.leaf_base);
     if (TRAV == 2) {  // esvo
+        f3 ro = add(p.cam.translation, splat(1.0f));
+        float t0, t1;
+        aabb_intersect(splat(1.0f), splat(2.0f), ro, rd, t0, t1);
+        ro = add(ro, smul(gmax(t0, 0.0f), rd));
+        if (TAGGED && !COUNT && p.stack_slots - 2u < kEsvoCellLevels) {  // 1 to kEsvoCellLevels levels
+            const EsvoRay r = esvo_setup(ro, rd);
+            if (esvo_cell_ray(ro, rd, r)) return fast_esvo_cells(fs, p.rec, p.stack_slots - 1u, p.cap, rd, r);
+        }
         float* stk_tmax = reinterpret_cast<float*>(stk_b);
         for (uint32_t s = 0; s < p.stack_slots; ++s) {
             stk_a[s * kWaveLanes] = 0u;
             stk_tmax[s * kWaveLanes] = 0.0f;
         }
-        f3 ro = add(p.cam.translation, splat(1.0f));
-        float t0, t1;
-        aabb_intersect(splat(1.0f), splat(2.0f), ro, rd, t0, t1);
-        ro = add(ro, smul(gmax(t0, 0.0f), rd));
-        if (TAGGED && !COUNT && p.rec)
-            return fast_esvo_rec(p.rec, p.leaf_base, p.cap, p.stack_slots, ro, rd, stk_a, stk_tmax);
         if (TAGGED && !COUNT) return fast_esvo(fs, p.cap, p.stack_slots, ro, rd, stk_a,
                                                 stk_tmax);
         if (TAGGED) return ref_esvo<COUNT>(TaggedNodes{p.cw, p.meta, p.node_count, p.index_mask, p.leaf_base}, p.cap, p.stack_slots, ro, rd, stk_a, stk_tmax,
