@@ -1,7 +1,8 @@
-"""The octree walks that take a short cut (esvo from cell to cell) against the
-general walk on the raw node words: trees at the edges of the short cut's range
-(1 level; the start table's 8 levels and one around them; the most levels and
-one more) and cameras that it must pass on or that meet cell borders exactly."""
+"""The octree walks that take a short cut (esvo from cell to cell, svo-df by the
+four children that a ray passes) against the general walk on the raw node words:
+trees at the edges of the short cuts' ranges (1 level; the start table's 8 levels
+and one around them; the most levels and one more) and cameras that they must
+pass on or that meet cell borders exactly."""
 import numpy as np
 import pytest
 
@@ -58,7 +59,7 @@ def _pair(ctx, nodes, side, t, cam, W=97, H=61):
 
 
 @pytest.mark.parametrize("depth", [1, 2, 7, 8, 9, 10, 14, 15])
-@pytest.mark.parametrize("t", [abi.ESVO])
+@pytest.mark.parametrize("t", [abi.ESVO, abi.SVO_DF])
 def test_chain_trees(ctx, t, depth):
     nodes = _chain_tree(depth, TARGET, seed=depth)
     lit = 0
@@ -71,7 +72,7 @@ def test_chain_trees(ctx, t, depth):
 
 @pytest.mark.parametrize("bad", [float("nan"), float("inf"), 1e30])
 @pytest.mark.parametrize("axis", [0, 2])
-@pytest.mark.parametrize("t", [abi.ESVO])
+@pytest.mark.parametrize("t", [abi.ESVO, abi.SVO_DF])
 def test_cameras_out_of_range(ctx, t, axis, bad):
     nodes = _chain_tree(9, TARGET, seed=3)
     eye = [0.4, 0.6, -0.8]
@@ -81,7 +82,7 @@ def test_cameras_out_of_range(ctx, t, axis, bad):
 
 
 @pytest.mark.parametrize("tree", [abi.TREE_DAG, abi.TREE_SPARSE])
-@pytest.mark.parametrize("t", [abi.ESVO])
+@pytest.mark.parametrize("t", [abi.ESVO, abi.SVO_DF])
 def test_built_trees(ctx, t, tree):
     """Every kind of leaf; the DAG has no records."""
     rng = np.random.default_rng(8)

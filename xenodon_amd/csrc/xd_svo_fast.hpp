@@ -481,57 +481,82 @@ __device__ __forceinline__ f3 fast_df(const FastSvo& s, uint64_t cap, uint32_t s
     return total;
 }
 
-// The walk of fast_df<true> on records.  It is bound by the instructions it
-// issues, half of the lanes busy, so it is built to need fewer trips:
+// The children that a ray passes in a node, in its order, and for how long.
+//
+// A line passes at most four of the eight: the near one first, then across the
+// middle planes in the order of their t.  With E the last near plane (0 at least),
+// X the first far plane and s1 <= s2 <= s3 the middle planes, child j's t-range is
+// [max(E, s_j), min(X, s_j+1)].  These are the floats of the box test, the greatest
+// near and the least far plane of the child's own six, since along each axis near
+// <= middle <= far after rounding as well; a child that crosses the planes in
+// another order has no length.  Of two equal middle planes either comes first: the
+// child between them has none.  All planes must be finite (df_ray).
+struct Passed {
+    float whole;            // of the node itself
+    float length[4];        // above 0 for a child that the box test hits
+    uint32_t axis1, axis3;  // index bits of the first and the last middle plane's axis
+};
+__device__ __forceinline__ Passed passed_children(const Planes& P) {
+    const float e = gmax(max_elem(mk(gmin(P.x0, P.x2), gmin(P.y0, P.y2), gmin(P.z0, P.z2))), 0.0f);
+    const float x = min_elem(mk(gmax(P.x0, P.x2), gmax(P.y0, P.y2), gmax(P.z0, P.z2)));
+    const f3 m = mk(P.x1, P.y1, P.z1);
+    const float s1 = min_elem(m), s2 = __builtin_amdgcn_fmed3f(m.x, m.y, m.z), s3 = max_elem(m);
+    Passed c;
+    c.whole = x - e;
+    c.length[0] = gmin(x, s1) - e;
+    c.length[1] = gmin(x, s2) - gmax(e, s1);
+    c.length[2] = gmin(x, s3) - gmax(e, s2);
+    c.length[3] = x - gmax(e, s3);
+    c.axis1 = m.x == s1 ? 4u : m.y == s1 ? 2u : 1u;
+    c.axis3 = m.x == s3 ? 4u : m.y == s3 ? 2u : 1u;
+    return c;
+}
+
+__device__ __forceinline__ bool df_ray(f3 rrd, f3 bias) {
+    return fabs_(bias.x) <= 1e30f && fabs_(bias.y) <= 1e30f && fabs_(bias.z) <= 1e30f && fabs_(rrd.x) <= 1e30f &&
+           fabs_(rrd.y) <= 1e30f && fabs_(rrd.z) <= 1e30f;
+}
+
+// The smaller key first.
+__device__ __forceinline__ void order(uint32_t& ka, float& a, uint32_t& kb, float& b) {
+    const bool swap = kb < ka;
+    const float f = swap ? b : a;
+    b = swap ? a : b;
+    a = f;
+    const uint32_t k = min(ka, kb);
+    kb = max(ka, kb);
+    ka = k;
+}
+
+// The walk of fast_df<true> on records, for rays that df_ray accepts.  It is bound
+// by the instructions it issues, half of the lanes busy, so it is built to need
+// fewer:
 //  * empty leaves, which add exactly +0, leave the hit mask at once;
-//  * a node without internal children -- most of the leaves with colour are
-//    under such -- is summed when it is entered: its eight colours are in its
-//    record and the box tests' bounds are the leaves' t-ranges, so there is no
-//    trip, no load and no t-range for a leaf;
-//  * a node that is finished when it is entered is popped, and the ancestor's
-//    next child taken, in the same trip.
-// Plain 1080p frames of a 512x361x512 volume: 1.82 / 1.92 / 5.92 -> 1.37 / 1.44
-// / 4.35 ms (outside / over it / inside).  Records alone, with a trip a leaf:
-// 1.71 / 1.71 / 5.57.  Summing such a node from its parent without entering it,
-// which saves the pop, was slower: 1.40 / 1.52 / 4.7.
-__device__ __forceinline__ f3 fast_df_rec(const uint4* __restrict__ rec, uint32_t n, uint64_t cap, f3 ro, f3 rd,
+//  * a trip takes one child, whatever it is: the planes of its box are a leaf's
+//    t-range, an internal node's hit test and the t-ranges of its children;
+//  * a node without internal children -- most of the leaves with colour are under
+//    such -- is summed from its parent, the four children that the ray passes in
+//    index order, so it costs no push and no pop;
+//  * a node that is finished is popped, and the ancestor's next child taken, in the
+//    same trip.
+// Plain 1080p frames of a 512x361x512 volume 1.22 / 1.40 / 4.20 -> 0.98 / 1.13 /
+// 3.33 ms, the three batched 6.12 -> 4.93, a 199x143 frame of a 128^3 volume 0.171
+// -> 0.138, against eight box tests a node and a sum in child order with each of the
+// eight under a condition.  Entering the nodes without internal children took 1.05 /
+// 1.18 / 3.43, and the head's load after the planes 1.05 / 1.14 / 3.39.
+__device__ __forceinline__ f3 fast_df_rec(const uint4* __restrict__ rec, uint32_t n, uint64_t cap, f3 rrd, f3 bias,
                                           uint32_t* stk_node, uint32_t* stk_child) {
-    f3 rrd = divv(splat(1.0f), rd);
-    f3 bias = mul(rrd, ro);
     int sp = 0;  // at most the tree's depth, below the stack's slots: each ancestor is on it once
-    uint32_t node = 0, depth = 0, mask = 0;
-    f3 corner = splat(0.0f);
-    float side = 0.5f;
     f3 total = splat(0.0f);
+    const uint32_t near = (rrd.x < 0.0f ? 4u : 0u) | (rrd.y < 0.0f ? 2u : 0u) | (rrd.z < 0.0f ? 1u : 0u), far = near ^ 7u;
     const uint32_t cap32 = cap32_of(cap);
     uint32_t it = 0;
-    NodeRec r;
-    bool enter = true;
+    // the root as the only child of a node around it
+    uint32_t node = 0, depth = ~0u, mask = 1;
+    f3 corner = splat(0.0f);
+    float side = 1.0f;  // of the node's children
+    NodeRec r = NodeRec{0u, (load_rec(rec_words(rec, 0)).masks & 0xFFu) ? 1u : 0x10001u};
     for (;;) {
-        if (enter) {
-            const GlobalWords w = rec_words(rec, node);
-            r = load_rec(w);
-            u32x4 c0 = *(const __attribute__((address_space(1))) u32x4*)(w + 4);
-            u32x4 c1 = *(const __attribute__((address_space(1))) u32x4*)(w + 8);
-            SlabPairs S = slab_pairs(node_planes(corner, side, rrd, bias));
-            // the three loads are in flight during the planes' arithmetic; without
-            // this the compiler issues them in turn, in the branches that use them
-            asm volatile(""
-                         : "+v"(r.inner), "+v"(r.masks), "+v"(c0), "+v"(c1), "+v"(S.xa0), "+v"(S.xb1), "+v"(S.ya0),
-                           "+v"(S.yb1), "+v"(S.za0), "+v"(S.zb1));
-            if ((r.masks & 0xFFu) == 0) {
-#pragma unroll
-                for (uint32_t k = 0; k < 8; ++k) {
-                    const uint32_t col = k < 4 ? c0[k & 3u] : c1[k & 3u];
-                    float lo, hi;
-                    slab_range(S, k, lo, hi);
-                    if (hi > lo && col != 0) total = add(total, muls(unorm_rgb(col), hi - lo));
-                }
-            } else {
-                mask = slab_hits(S) & (r.masks | (r.masks >> 8)) & 0xFFu;
-            }
-            enter = false;
-        }
         if (mask == 0) {
             if (sp == 0) break;
             --sp;
@@ -551,26 +576,49 @@ __device__ __forceinline__ f3 fast_df_rec(const uint4* __restrict__ rec, uint32_
         if (++it > cap32) break;
         const uint32_t rest = mask & (mask - 1u), bit = mask ^ rest;
         mask = rest;
-        if (r.masks & (bit << 8)) {
-            const uint32_t ci = (uint32_t)__builtin_ctz(bit);
-            const uint32_t col = rec_words(rec, node)[4 + ci];
-            float t_min, t_max;
-            child_trange(corner, side, rrd, bias, ci, t_min, t_max);
-            total = add(total, muls(unorm_rgb(col), t_max - gmax(t_min, 0.0f)));
+        const bool leaf = (r.masks & (bit << 8)) != 0;
+        const uint32_t child = leaf ? node : r.inner + __popc(r.masks & (bit - 1u) & 0xFFu);
+        const GlobalWords w = rec_words(rec, child);
+        NodeRec next = load_rec(w);  // in flight during the planes' arithmetic; wanted by an internal node
+        const f3 at = mk((bit & 0xF0u) ? corner.x + side : corner.x, (bit & 0xCCu) ? corner.y + side : corner.y,
+                         (bit & 0xAAu) ? corner.z + side : corner.z);
+        Passed c = passed_children(node_planes(at, side * 0.5f, rrd, bias));
+        asm volatile(""
+                     : "+v"(next.inner), "+v"(next.masks), "+v"(c.length[0]), "+v"(c.length[1]), "+v"(c.length[2]),
+                       "+v"(c.length[3]));
+        if (leaf) {
+            total = add(total, muls(unorm_rgb(w[4 + __builtin_ctz(bit)]), c.whole));
+        } else if (r.masks & (bit << 16)) {
+            uint32_t k0 = near, k1 = near ^ c.axis1, k2 = far ^ c.axis3, k3 = far;
+            order(k0, c.length[0], k1, c.length[1]);
+            order(k2, c.length[2], k3, c.length[3]);
+            order(k0, c.length[0], k2, c.length[2]);
+            order(k1, c.length[1], k3, c.length[3]);
+            order(k1, c.length[1], k2, c.length[2]);
+            // 0 for empty leaves; a child not passed adds +0
+            const uint32_t col[4] = {w[4 + k0], w[4 + k1], w[4 + k2], w[4 + k3]};
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j) total = add(total, muls(unorm_rgb(col[j]), gmax(c.length[j], 0.0f)));
         } else {
-            if (mask != 0) {
+            if (rest != 0) {
                 stk_node[sp * kWaveLanes] = node;
-                stk_child[sp * kWaveLanes] = mask | (depth << 8);
+                stk_child[sp * kWaveLanes] = rest | (depth << 8);
                 ++sp;
             }
-            node = r.inner + __popc(r.masks & (bit - 1u) & 0xFFu);
-            corner = mk((bit & 0xF0u) ? corner.x + side : corner.x, (bit & 0xCCu) ? corner.y + side : corner.y,
-                        (bit & 0xAAu) ? corner.z + side : corner.z);
+            r = next;
+            node = child;
+            corner = at;
             side = side * 0.5f;
             depth = depth + 1u;
-            mask = 0;
-            enter = true;
+            mask = (c.length[0] > 0.0f ? 1u << near : 0u) | (c.length[1] > 0.0f ? 1u << (near ^ c.axis1) : 0u) |
+                   (c.length[2] > 0.0f ? 1u << (far ^ c.axis3) : 0u) | (c.length[3] > 0.0f ? 1u << far : 0u);
+            mask &= (r.masks | (r.masks >> 8)) & 0xFFu;
         }
+        // One way back to the top: else the compiler makes a loop of its own of the
+        // ways that leave the node as it is, and the lanes in it keep the others waiting
+        // (1.35 / 1.71 / 4.32 ms).
+        pin(corner);
+        asm volatile("" : "+v"(mask), "+v"(node), "+v"(side));
     }
     return total;
 }

@@ -295,8 +295,10 @@ __device__ __forceinline__ f3 svo_pixel(const RenderParams& p, f3 rd, uint32_t* 
     }
     const f3 ro = p.cam.translation;
     if (TRAV == 3) {  // svo-df
-        if (TAGGED && !COUNT && p.rec)
-            return fast_df_rec(p.rec, p.leaf_base, p.cap, ro, rd, stk_a, stk_b);
+        if (TAGGED && !COUNT && p.rec) {
+            const f3 rrd = divv(splat(1.0f), rd), bias = mul(rrd, ro);
+            if (df_ray(rrd, bias)) return fast_df_rec(p.rec, p.leaf_base, p.cap, rrd, bias, stk_a, stk_b);
+        }
         if (TAGGED && !COUNT)  // depth-field handling fixed per tree (a uniform choice)
             return p.depth_exact ? fast_df<true>(fs, p.cap, p.stack_slots, ro, rd, stk_a, stk_b)
                                  : fast_df<false>(fs, p.cap, p.stack_slots, ro, rd, stk_a, stk_b);
