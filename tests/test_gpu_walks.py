@@ -1,11 +1,12 @@
-"""The octree walks that take a short cut (esvo from cell to cell, svo-df by the
-four children that a ray passes) against the general walk on the raw node words:
+"""The octree walks that take a short cut (esvo and svo-rope from cell to cell,
+svo-df by the four children that a ray passes) against the general walk on the raw node words:
 trees at the edges of the short cuts' ranges (1 level; the start table's 8 levels
 and one around them; the most levels and one more) and cameras that they must
 pass on or that meet cell borders exactly."""
 import numpy as np
 import pytest
 
+from oracle import xo
 from tests.test_gpu_parity import _chain_tree
 from xenodon_amd import abi
 
@@ -58,10 +59,17 @@ def _pair(ctx, nodes, side, t, cam, W=97, H=61):
     return images
 
 
-@pytest.mark.parametrize("depth", [1, 2, 7, 8, 9, 10, 14, 15])
-@pytest.mark.parametrize("t", [abi.ESVO, abi.SVO_DF])
+def _tree(depth, t, seed):
+    nodes = _chain_tree(depth, TARGET, seed=seed)
+    if t == abi.SVO_ROPE:
+        xo.lib().xo_generate_ropes(nodes.ctypes.data, nodes.shape[0], 1 << depth)
+    return nodes
+
+
+@pytest.mark.parametrize("depth", [1, 2, 7, 8, 9, 10, 12, 13, 14, 15])
+@pytest.mark.parametrize("t", [abi.ESVO, abi.SVO_DF, abi.SVO_ROPE])
 def test_chain_trees(ctx, t, depth):
-    nodes = _chain_tree(depth, TARGET, seed=depth)
+    nodes = _tree(depth, t, seed=depth)
     lit = 0
     for name, cam in CAMERAS.items():
         got, want = _pair(ctx, nodes, 1 << depth, t, cam())
@@ -72,24 +80,64 @@ def test_chain_trees(ctx, t, depth):
 
 @pytest.mark.parametrize("bad", [float("nan"), float("inf"), 1e30])
 @pytest.mark.parametrize("axis", [0, 2])
-@pytest.mark.parametrize("t", [abi.ESVO, abi.SVO_DF])
+@pytest.mark.parametrize("t", [abi.ESVO, abi.SVO_DF, abi.SVO_ROPE])
 def test_cameras_out_of_range(ctx, t, axis, bad):
-    nodes = _chain_tree(9, TARGET, seed=3)
+    nodes = _tree(9, t, seed=3)
     eye = [0.4, 0.6, -0.8]
     eye[axis] = bad
     got, want = _pair(ctx, nodes, 512, t, _camera(eye, (0.1, 0.05, 1.0)), 33, 17)
     assert np.array_equal(got, want)
 
 
-@pytest.mark.parametrize("tree", [abi.TREE_DAG, abi.TREE_SPARSE])
-@pytest.mark.parametrize("t", [abi.ESVO, abi.SVO_DF])
-def test_built_trees(ctx, t, tree):
-    """Every kind of leaf; the DAG has no records."""
+def _grid():
     rng = np.random.default_rng(8)
     grid = rng.integers(0, 256, (24, 24, 24, 4), dtype=np.uint8)
     grid[rng.random((24, 24, 24)) < 0.6] = 0
-    grid = np.kron(grid, np.ones((2, 2, 2, 1), np.uint8))
-    nodes, st = abi.build_octree(grid, tree=tree)
+    return np.kron(grid, np.ones((2, 2, 2, 1), np.uint8))
+
+
+@pytest.mark.parametrize("t, tree", [(abi.ESVO, abi.TREE_DAG), (abi.ESVO, abi.TREE_SPARSE), (abi.SVO_DF, abi.TREE_DAG),
+                                     (abi.SVO_DF, abi.TREE_SPARSE), (abi.SVO_ROPE, abi.TREE_ROPE),
+                                     (abi.SVO_ROPE, abi.TREE_SPARSE)])
+def test_built_trees(ctx, t, tree):
+    """Every kind of leaf; the DAG has no records, the sparse tree no ropes."""
+    nodes, st = abi.build_octree(_grid(), tree=tree)
     for name, cam in CAMERAS.items():
         got, want = _pair(ctx, nodes, st["side"], t, cam())
+        assert np.array_equal(got, want), name
+
+
+@pytest.mark.parametrize("depth", [8, 10])
+@pytest.mark.parametrize("change", ["cut", "turned", "deeper", "higher", "depth"])
+def test_changed_ropes(ctx, change, depth):
+    """Ropes that do not lead where the geometry says are followed as they are."""
+    if depth == 8:  # the grid in a corner of 256^3 voxels
+        grid = np.zeros((48, 48, 129, 4), np.uint8)
+        grid[:, :, 1:49] = _grid()
+        grid[:, :, 128] = 77
+        nodes, st = abi.build_octree(grid, tree=abi.TREE_ROPE)
+        nodes, side = nodes.copy(), st["side"]
+        assert side == 256
+    else:
+        nodes, side = _tree(depth, abi.SVO_ROPE, seed=5), 1 << depth
+    leaf = nodes[:, 9] >= 1 << 31
+    parent = np.zeros(len(nodes), np.int64)
+    for k in range(8):
+        parent[nodes[~leaf, k]] = np.nonzero(~leaf)[0]
+    where = np.nonzero(leaf[:, None] & (nodes[:, :6] != 0))
+    pick = np.random.default_rng(2).choice(len(where[0]), max(1, len(where[0]) // 7), replace=False)
+    for i, k in zip(where[0][pick], where[1][pick]):
+        to = nodes[i, k]
+        if change == "cut":
+            nodes[i, k] = 0
+        elif change == "turned":
+            nodes[i, k] = nodes[i, (k + 2) % 6]
+        elif change == "deeper" and not leaf[to]:
+            nodes[i, k] = nodes[to, 3]
+        elif change == "higher" and parent[to]:
+            nodes[i, k] = parent[to]
+        elif change == "depth":
+            nodes[i, 9] = (nodes[i, 9] & 0x80000000) | max(1, int(nodes[i, 9] & 0xFF) - 1)
+    for name, cam in CAMERAS.items():
+        got, want = _pair(ctx, nodes, side, abi.SVO_ROPE, cam(), 41, 29)
         assert np.array_equal(got, want), name

@@ -47,6 +47,10 @@ constexpr uint64_t kTableBytes = kTableCells * 8;
 // The entry's second word: the level, and whether the node is internal with only
 // leaves for children and has a record.
 constexpr uint32_t kTableLevelMask = 0xFFu, kTableLowNode = 0x100u;
+// Levels of the trees whose ropes the upload checks: from the table's, as
+// shallower ones keep to their ropes (see fill_params), to where a thread, which
+// checks the leaves below a table cell, has 8^4 of them.
+constexpr uint32_t kRopeCellFirst = kTableLevel, kRopeCellLast = 12;
 constexpr uint32_t kRecWords = 12;  // words of an internal node's record (RenderParams::rec)
 
 // Everything one traversal launch needs; passed by value as the kernel
@@ -94,6 +98,7 @@ struct RenderParams {
     // RGB (0 for all but leaves)}.  A node's internal children have
     // consecutive indices, so one index and a mask name them all.
     const uint4* rec;
+    uint32_t rope_cells;  // svo-rope goes by the table: the ropes and depth fields are those of the tree's geometry
     uint32_t xcd_chunks;  // plain launches: block runs per XCD (0: hardware order)
     unsigned long long* words;  // word counter (instrumented variant only)
 };

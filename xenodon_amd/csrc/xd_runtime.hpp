@@ -63,6 +63,7 @@ struct xd_volume {
     uint32_t root_tag = 0;
     uint32_t depth_exact = 0;  // internal nodes' depth fields match their depth (see octree_depths_exact)
     uint32_t top[xd::kTopLevels] = {0, 0, 0, 0};  // nodes in breadth-first levels 0..L
+    bool rope_cells = false;   // every rope leads where the tree's geometry says (see RenderParams::rope_cells)
     bool one_block = false;    // d_meta and d_table are parts of d_cw's allocation
     uint64_t rec_at = 0;       // word of d_cw where the internal nodes' records begin (0: none, see RenderParams::rec)
     uint32_t leaf_base = 0;    // tagged layout: first leaf; the leaves' ropes are stored as planes

@@ -311,6 +311,8 @@ __device__ __forceinline__ f3 svo_pixel(const RenderParams& p, f3 rd, uint32_t* 
         return ref_naive<COUNT>(RawNodes{p.nodes, p.node_count}, p.cap, ro, rd, words);
     }
     // svo-rope
+    if (TAGGED && !COUNT && p.rope_cells && rope_cell_ray(ro, rd))
+        return fast_rope_cells(fs, p.rec, p.cap, ro, rd);
     if (TAGGED && !COUNT) return fast_rope(fs, p.cap, ro, rd);
     if (TAGGED) return ref_rope<COUNT>(TaggedNodes{p.cw, p.meta, p.node_count, p.index_mask, p.leaf_base}, p.cap, ro, rd, words);
     return ref_rope<COUNT>(RawNodes{p.nodes, p.node_count}, p.cap, ro, rd, words);
