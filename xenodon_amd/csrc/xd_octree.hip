@@ -316,13 +316,21 @@ __global__ __launch_bounds__(kOctBlock) void k_oct_emit(const uint2* __restrict_
 // One cell of the start table a thread: the walk of build_start_table.
 // stop: null, or a word that says, when set, that the child words are no tree's.
 __global__ __launch_bounds__(256) void k_start_table(const uint32_t* __restrict__ cw, uint32_t root_tag,
-                                                     uint32_t index_mask, const uint4* __restrict__ rec,
-                                                     const uint32_t* stop, uint2* __restrict__ table) {
+                                                     uint32_t index_mask, uint32_t shift,
+                                                     const uint4* __restrict__ rec, const uint32_t* stop,
+                                                     uint2* __restrict__ table) {
     if (stop && *stop) return;
-    const uint32_t cell = blockIdx.x * 256 + threadIdx.x;
-    const uint3 p = table_place(cell);
+    uint32_t cell = blockIdx.x * 256 + threadIdx.x;
+    const uint32_t levels = kTableLevel - shift;
+    uint3 p = table_place(cell);
+    if (shift) {  // the cells below 2^levels of each axis
+        const uint32_t m = (1u << levels) - 1u, sh = 23u - levels;
+        if (cell >> (3 * levels)) return;
+        p = make_uint3((cell & m) << sh, (cell >> levels & m) << sh, (cell >> (2 * levels) & m) << sh);
+        cell = table_cell(p.x >> shift, p.y >> shift, p.z >> shift);
+    }
     uint32_t word = root_tag, level = 0;
-    while (!(word & kTagLeaf) && level < kTableLevel) {
+    while (!(word & kTagLeaf) && level < levels) {
         const uint32_t s = 22u - level;
         const uint32_t k = (p.x >> s & 1u) << 2 | (p.y >> s & 1u) << 1 | (p.z >> s & 1u);
         word = cw[(uint64_t)(word & index_mask) * 8 + k];
@@ -395,10 +403,10 @@ __global__ __launch_bounds__(256) void k_check_ropes(const uint32_t* __restrict_
     }
 }
 
-hipError_t launch_start_table(const uint32_t* cw, uint32_t root_tag, uint32_t index_mask, const uint4* rec,
+hipError_t launch_start_table(const uint32_t* cw, uint32_t root_tag, uint32_t index_mask, uint32_t shift, const uint4* rec,
                               const uint32_t* stop, uint2* table, hipStream_t s) {
-    hipLaunchKernelGGL(k_start_table, dim3((uint32_t)(kTableCells / 256)), dim3(256), 0, s, cw, root_tag, index_mask,
-                       rec, stop, table);
+    hipLaunchKernelGGL(k_start_table, dim3((uint32_t)(((kTableCells >> (3 * shift)) + 255) / 256)), dim3(256), 0, s, cw,
+                       root_tag, index_mask, shift, rec, stop, table);
     return hipGetLastError();
 }
 
@@ -500,7 +508,7 @@ bool derive_layout_on_device(xd_volume* v, const uint32_t* w, uint64_t n, bool w
             return hipGetLastError();
         };
         if ((e = hipGetLastError()) != hipSuccess ||
-            (e = launch_start_table(v->d_cw, v->root_tag, index_mask, root_leaf ? nullptr : rec, &flags->twice, v->d_table, s)) != hipSuccess ||
+            (e = launch_start_table(v->d_cw, v->root_tag, index_mask, table_shift_of(max_depth), root_leaf ? nullptr : rec, &flags->twice, v->d_table, s)) != hipSuccess ||
             (check_ropes && (e = launch_check_ropes()) != hipSuccess) ||
             (e = hipMemcpyAsync(&f, flags, sizeof(f), hipMemcpyDeviceToHost, s)) != hipSuccess ||
             (e = hipStreamSynchronize(s)) != hipSuccess)

@@ -117,6 +117,7 @@ void fill_params(RenderParams& p, const xd_volume* vol, int traversal, const xd_
         p.cw = vol->d_cw;
         p.meta = vol->d_meta;
         p.table = vol->d_table;
+        p.table_shift = table_shift_of(vol->max_depth);
         p.rope_depth = vol->rope_depth;
         p.index_mask = vol->index_mask;
         p.empty_tag = vol->empty_tag;
@@ -673,7 +674,7 @@ int xd_volume_from_svo(xd_context* ctx, const void* nodes, uint64_t node_count, 
         const uint32_t root_ld = w[9], root_col = w[8];
         v->root_tag = (root_ld & kLeafMask) ? (kTagLeaf | ((root_col & 0xFFFFFFu) ? 0u : v->empty_tag)) : 0u;
         if ((e = hipMalloc(&v->d_table, kTableBytes)) != hipSuccess ||
-            (e = launch_start_table(v->d_cw, v->root_tag, v->index_mask, nullptr, nullptr, v->d_table, ctx->stream)) != hipSuccess ||
+            (e = launch_start_table(v->d_cw, v->root_tag, v->index_mask, table_shift_of(v->max_depth), nullptr, nullptr, v->d_table, ctx->stream)) != hipSuccess ||
             (e = hipStreamSynchronize(ctx->stream)) != hipSuccess) {
             xd_volume_free(v);
             return fail_hip(e, "octree upload");

@@ -134,7 +134,7 @@ void build_start_table(const uint32_t* child_w, uint32_t root_tag, uint32_t inde
 // The device's table, built there from the device form of child_w: the same
 // entries in the order of table_cell, with kTableLowNode from rec (or null).  stop:
 // null, or a device word that, if set, keeps the table unwritten.
-hipError_t launch_start_table(const uint32_t* cw, uint32_t root_tag, uint32_t index_mask, const uint4* rec,
+hipError_t launch_start_table(const uint32_t* cw, uint32_t root_tag, uint32_t index_mask, uint32_t shift, const uint4* rec,
                               const uint32_t* stop, uint2* table, hipStream_t s);
 // Derives v's tagged layout and start table on the device from n .svo nodes in
 // host memory, and sets everything of v that depends on them.  False if the

@@ -31,6 +31,7 @@ struct FastSvo {
     uint32_t n;            // node count (indices read back from a stack are clamped to it)
     uint32_t depth_exact;  // depth fields of internal nodes equal their tree depth
     const uint2* table;    // start table: kTableCells entries {child word, level}, or null
+    uint32_t table_shift;  // ... of cells coarser by this many levels
     uint32_t rope_depth;   // ropes carry their targets' depth fields (kRopeDepthShift)
     uint32_t index_mask;   // index bits of a child word
     // a child word wd names an empty leaf iff (wd & empty_mask) >= empty_min:
@@ -63,9 +64,9 @@ __device__ __forceinline__ bool empty_leaf(const FastSvo& s, uint32_t wd) { retu
 // index range from empty_start on.  One comparison covers both.
 __device__ __forceinline__ FastSvo make_fast_svo(const uint32_t* cw, const uint32_t* meta, uint32_t root_tag,
                                                  const uint32_t* top, uint32_t n_top, uint32_t n, uint32_t depth_exact,
-                                                 const uint2* table, uint32_t rope_depth, uint32_t index_mask,
+                                                 const uint2* table, uint32_t table_shift, uint32_t rope_depth, uint32_t index_mask,
                                                  uint32_t empty_tag, uint32_t empty_start, uint32_t leaf_base) {
-    return FastSvo{cw, meta, root_tag, top, n_top, n, depth_exact, table, rope_depth, index_mask,
+    return FastSvo{cw, meta, root_tag, top, n_top, n, depth_exact, table, table_shift, rope_depth, index_mask,
                    empty_tag ? empty_tag : index_mask, empty_tag ? empty_tag : empty_start, leaf_base};
 }
 
@@ -127,6 +128,19 @@ __device__ __forceinline__ uint3 table_place(uint32_t cell) {
                       (cell >> (2 * b + 6) & m) << (sh + 2) | (cell >> 4 & 3u) << sh);
 }
 
+// The index in s's table.  A branch that all lanes take alike: three shifts by 0 in
+// each step of a ray had cost the walks 3 to 4 % on a 9-level tree.
+__device__ __forceinline__ uint32_t table_index(const FastSvo& s, uint32_t x, uint32_t y, uint32_t z) {
+    uint32_t at;
+    if (s.table_shift == 0) {
+        at = table_cell(x, y, z);
+    } else {
+        at = table_cell(x >> s.table_shift, y >> s.table_shift, z >> s.table_shift);
+        asm volatile("" : "+v"(at));  // or the compiler makes one computation of the two again
+    }
+    return at;
+}
+
 // svo_naive.comp:8-27 with tagged pointers.  `tag` returns the found node's
 // tags.  With a start table the walk begins at the node the table holds for
 // the point's level-kTableLevel cell (found from the point's level bits): the same node
@@ -140,7 +154,7 @@ __device__ __forceinline__ uint32_t fast_find(const FastSvo& s, f3 pos, f3& base
     tag = s.root_tag;
     if (s.table) {
         const uint32_t bx = level_bits(pos.x), by = level_bits(pos.y), bz = level_bits(pos.z);
-        const uint2 e = s.table[table_cell(bx, by, bz)];
+        const uint2 e = s.table[table_index(s, bx, by, bz)];
         index = e.x & s.index_mask;
         tag = e.x;
         level = e.y & kTableLevelMask;
@@ -264,7 +278,7 @@ __device__ __forceinline__ f3 fast_naive(const FastSvo& s, const uint4* __restri
         if (++it > cap32) break;
         const f3 pt = add(smul(t, rd), ro);
         const uint32_t bx = level_bits(pt.x), by = level_bits(pt.y), bz = level_bits(pt.z);
-        const uint32_t at = table_cell(bx, by, bz);
+        const uint32_t at = table_index(s, bx, by, bz);
         if (at != cell) {
             e = s.table[at];
             cell = at;
@@ -765,7 +779,7 @@ __device__ __forceinline__ f3 fast_rope_cells(const FastSvo& s, const uint4* __r
         const uint32_t bx = clamp3(floor_bits(pos.x), nx, nx | rest);
         const uint32_t by = clamp3(floor_bits(pos.y), ny, ny | rest);
         const uint32_t bz = clamp3(floor_bits(pos.z), nz, nz | rest);
-        const uint2 e = s.table[table_cell(bx, by, bz)];
+        const uint2 e = s.table[table_index(s, bx, by, bz)];
         total = add(total, muls(unorm_rgb(pend_col), pend_w));  // +0 the first time
         pin(total);
         const uint32_t* colour;
@@ -930,7 +944,7 @@ __device__ __forceinline__ f3 fast_esvo_cells(const FastSvo& s, const uint4* __r
         const int32_t cy = esvo_cell(q, t_min, nd.y, r.t_coeff.y, r.t_bias.y, ny, rest);
         const int32_t cz = esvo_cell(q, t_min, nd.z, r.t_coeff.z, r.t_bias.z, nz, rest);
         const uint32_t bx = (uint32_t)cx ^ fx, by = (uint32_t)cy ^ fy, bz = (uint32_t)cz ^ fz;
-        const uint2 e = s.table[table_cell(bx, by, bz)];
+        const uint2 e = s.table[table_index(s, bx, by, bz)];
         total = add(total, muls(unorm_rgb(pend_col), pend_w));  // +0 the first time
         pin(total);
         const uint32_t* colour;
