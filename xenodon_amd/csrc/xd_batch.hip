@@ -7,9 +7,9 @@
 // class (by default, its waves starting on different classes so that each CU
 // runs latency-bound and issue-bound traversals side by side), or each class
 // gets a kernel with the registers and LDS of its own traversal only.  Within
-// a class the tiles are dealt into 8 ranges by the band of the view they lie
-// in, one range per XCD (the hardware deals workgroups to the XCDs
-// round-robin, so block b runs on XCD b % 8).  A wavefront takes tiles from
+// a class the tiles are dealt in squares to 8 ranges in turn, one range per
+// XCD (the hardware deals workgroups to the XCDs round-robin, so block b runs
+// on XCD b % 8).  A wavefront takes tiles from
 // its own XCD's range with one atomic per grab, and when that range is
 // exhausted it moves on to the other ranges, so a kernel ends only when every
 // tile of its classes is done and no CU idles while work is left.  Each tile

@@ -4,15 +4,14 @@
 // operation in FP32, so that frames are bit-identical to the CPU restatement
 // of the same shader.  Shortcuts are taken only where they cannot change a
 // result: a texel whose RGB is zero adds exactly +0 to the sum, so the DDA
-// skips the fetch of voxels in bricks known to be empty (the side-distance
+// skips the fetch of voxels with no colour in reach (the side-distance
 // additions, which decide the voxel sequence, still run for every step).
 //
 // Work decomposition: a 256-thread block is four wavefronts; each wavefront
 // takes one 8x8 (or 16x4 / 32x2) pixel tile, so a wave's rays start together
 // and walk neighbouring voxels/nodes (coherent gathers through L2).  The
-// hardware deals blocks to the 8 XCDs round-robin; blocks are renumbered so
-// each XCD renders one contiguous band of the image and its L2 keeps that
-// band's part of the volume.
+// hardware deals blocks to the 8 XCDs round-robin, and by default neighbouring
+// blocks stay on different XCDs (see block_pixel).
 #include "xd_trace.hpp"
 
 namespace xd {

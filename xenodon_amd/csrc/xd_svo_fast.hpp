@@ -6,8 +6,10 @@
 // Trees above 2^30 nodes carry 31-bit indices and no empty tag; their empty
 // leaves are the indices from a threshold on (empty_mask and empty_min of
 // FastSvo cover both).
-// The traversal arithmetic is the shaders' (see xd_svo_ref.hpp); only loads
-// change:
+// Two kinds of walk.  The general ones (fast_df, fast_esvo, fast_rope) take the
+// shaders' steps (see xd_svo_ref.hpp) and change only the loads; fast_naive,
+// fast_esvo_cells, fast_rope_cells and fast_df_rec take other steps to the same
+// leaves, and say why every float that reaches a sum is the shader's.  In both:
 //   * "is this node a leaf?" comes with the pointer that led to it, so a
 //     descent costs one dependent load per level instead of two;
 //   * the colour of an empty leaf is known to be 0 without a load (the sum
