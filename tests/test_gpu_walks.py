@@ -141,3 +141,50 @@ def test_changed_ropes(ctx, change, depth):
     for name, cam in CAMERAS.items():
         got, want = _pair(ctx, nodes, side, abi.SVO_ROPE, cam(), 41, 29)
         assert np.array_equal(got, want), name
+
+
+def _corner_tree(depth):
+    """A rope tree of blocky voxels in a corner of 2^depth voxels a side, with leaves above the start table's level
+    beside regions that reach down to it."""
+    block = _grid() if depth == 8 else np.kron(_grid(), np.ones((2, 2, 2, 1), np.uint8))
+    size, half = block.shape[0], 1 << (depth - 1)
+    grid = np.zeros((size, size, half + 1, 4), np.uint8)
+    grid[:, :, :size] = block
+    grid[:, :, half] = 77
+    nodes, st = abi.build_octree(grid, tree=abi.TREE_ROPE)
+    assert st["side"] == 1 << depth
+    return nodes.copy(), st["side"], size / st["side"]
+
+
+@pytest.mark.parametrize("depth", [8, 10])
+@pytest.mark.parametrize("to", ["child", "between", "corner"])
+def test_ropes_into_the_near_corner_of_their_target(ctx, to, depth):
+    """A rope that leads to a descendant at its target's lower corner, which the place beside the leaf is in as well,
+    ends in that descendant wherever the ray goes on."""
+    nodes, side, used = _corner_tree(depth)
+    plain = nodes.copy()
+    leaf = nodes[:, 9] >= 1 << 31
+    turned = 0
+    for i, k in zip(*np.nonzero(leaf[:, None] & (nodes[:, :6] != 0))):
+        chain = [nodes[i, k]]
+        while not leaf[chain[-1]]:
+            chain.append(nodes[chain[-1], 0])
+        if nodes[chain[-1], 9] & 0xFF > 8:  # below the table: the place's entry is none of the chain's leaves
+            continue
+        if to == "between":
+            pick = 1 + len(chain[1:-1]) // 2 if len(chain) > 3 else 0
+        else:
+            pick = min(1, len(chain) - 1) if to == "child" else len(chain) - 1
+        nodes[i, k] = chain[pick]
+        turned += pick > 0
+    assert turned > 20
+    mid = 0.5 * used
+    near = [_camera((-0.8 * used, 1.4 * used, -1.1 * used), np.array([mid] * 3) - np.array((-0.8, 1.4, -1.1)) * used),
+            _camera((2.1 * used, -0.7 * used, 1.3 * used), np.array([mid] * 3) - np.array((2.1, -0.7, 1.3)) * used),
+            _camera((0.4 * used, 0.45 * used, 0.7 * used), (1.0, -0.7, -0.4))]
+    changed = 0
+    for cam in near + [make() for make in CAMERAS.values()]:
+        got, want = _pair(ctx, nodes, side, abi.SVO_ROPE, cam, 41, 29)
+        changed += int((want != _pair(ctx, plain, side, abi.SVO_ROPE, cam, 41, 29)[1]).any())
+        assert np.array_equal(got, want), int((got != want).any(-1).sum())
+    assert changed  # or the ropes would not matter to these views

@@ -347,10 +347,10 @@ __global__ __launch_bounds__(256) void k_start_table(const uint32_t* __restrict_
 // go from leaf to leaf by position (fast_rope_cells).  A rope's target is the node
 // beside the leaf at the leaf's level, or the leaf that holds that place; the table
 // knows the place's leaf or its level-8 node, and whichever of the two is the
-// higher must lead down to the other.  A thread takes the leaves of one table cell:
-// those above it if the cell is their first, else all below its node.  (A 1.3 M
-// node load with its first frame, of which the rope walk is 0.1 ms less, 2.71 ->
-// 2.75 ms.)
+// higher must lead down to the other, in as many steps as there are levels between.
+// A thread takes the leaves of one table cell: those above it if the cell is their
+// first, else all below its node.  (A 1.3 M node load with its first frame, of which
+// the rope walk is 0.1 ms less, 2.71 -> 2.75 ms.)
 __global__ __launch_bounds__(256) void k_check_ropes(const uint32_t* __restrict__ cw, const uint32_t* __restrict__ meta,
                                                      uint32_t n, uint32_t leaf_base, uint32_t index_mask,
                                                      uint32_t depth, const uint2* __restrict__ table, OctFlags* flags) {
@@ -391,10 +391,15 @@ __global__ __launch_bounds__(256) void k_check_ropes(const uint32_t* __restrict_
             uint32_t at = e.y & kTableLevelMask, a = e.x, b = rope;
             if (at <= level) {  // from the table's node down to the leaf's level
                 for (; at < level && !(a & kTagLeaf); ++at) a = step(a, at, q);
-            } else {  // from the rope's target, at the leaf's level, down to the table's node
-                for (uint32_t l = level; l < at && !(b & kTagLeaf); ++l) b = step(b, l, q);
+            } else {
+                // from the rope's target, at the leaf's level, down to the table's node, each
+                // level in between: a descendant of the target at the place's corner leads to
+                // that node too, by fewer
+                uint32_t l = level;
+                for (; l < at && !(b & kTagLeaf); ++l) b = step(b, l, q);
+                bad = l != at;
             }
-            bad = ((a ^ b) & index_mask) != 0;
+            bad |= ((a ^ b) & index_mask) != 0;
         }
         if (bad) {
             flags->bad_rope = 1;
