@@ -140,3 +140,16 @@ def test_malformed_nodes_are_refused(ctx):
         with pytest.raises(abi.XdError) as err:
             ctx.svo_volume(nodes, 64)
         assert err.value.status == abi.XD_ERR_FORMAT
+
+
+@pytest.mark.parametrize("level", [0, 1, 2])
+def test_internal_children_named_twice_near_the_root(ctx, level):
+    """All children of a node of the first levels are one internal child, the others and what is below them named by
+    none: a node count that a tree could have, but more child words to number than there are nodes."""
+    nodes = random_tree(600, seed=1)
+    inner = (nodes[:, 9] & LEAF) == 0
+    p = 0
+    for _ in range(level):
+        p = next(int(c) for c in nodes[p, :8] if inner[c])
+    nodes[p, :8] = next(int(c) for c in nodes[p, :8] if inner[c])
+    _same(ctx, nodes)

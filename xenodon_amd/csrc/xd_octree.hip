@@ -428,6 +428,9 @@ bool derive_layout_on_device(xd_volume* v, const uint32_t* w, uint64_t n, bool w
         for (uint32_t old : level) {
             const uint32_t* nd = w + (uint64_t)old * kNodeWords;
             if (nd[9] & kLeafMask) continue;
+            // named twice, its children would be counted twice and the indices run past the nodes
+            for (const uint4& t : top)
+                if (t.x == old) return false;
             top.push_back(make_uint4(old, count[0], count[1], count[2]));
             for (int k = 0; k < 8; ++k) {
                 if (nd[k] >= n) return false;
@@ -483,8 +486,13 @@ bool derive_layout_on_device(xd_volume* v, const uint32_t* w, uint64_t n, bool w
             (e = hipMemcpyAsync(&f, flags, sizeof(f), hipMemcpyDeviceToHost, s)) != hipSuccess ||
             (e = hipStreamSynchronize(s)) != hipSuccess)
             break;
-        // every node but the root is a child once: 1 + 8 * internal nodes, none of them twice
+        // every node but the root is a child once: 1 + 8 * internal nodes, none of them twice.
+        // The children numbered are as many as the nodes then, and every index k_oct_number
+        // and k_oct_emit make is below n, also where a node further down is named twice.
         if (f.refused || 1 + 8ull * f.total[3] != n) break;
+        uint64_t numbered = 0;
+        for (int q = 0; q < 3; ++q) numbered += (uint64_t)count[q] + f.total[q];
+        if (numbered != n) break;
         const uint32_t max_depth = f.total[3] ? f.inner_depth + 1 : 0;
         if (max_depth > 23) break;
         OctBases B;
