@@ -60,3 +60,21 @@ def test_std_dev_limit_reached_exactly(ctx):
         got, gst = ctx.build_octree(gv, heuristic=abi.HEURISTIC_STD_DEV, std_dev=float(sd))
         assert gst == wst and np.array_equal(got, want), sd
     gv.free()
+
+
+# x, y, z: a node of the upper levels is mostly outside of these
+THIN = [(2, 4099, 4), (1, (1 << 17) + 1, 6), (70000, 3, 2), (5, 1, 1 << 18), (1, 1030, 517)]
+
+
+@pytest.mark.parametrize("dims", THIN)
+def test_std_dev_of_thin_grids(ctx, dims):
+    """The sums take the grid's part of a node, not the side^3 of all of it."""
+    x, y, z = dims
+    grid = np.random.default_rng(x + y).integers(0, 256, (z, y, x, 4), dtype=np.uint8)
+    gv = ctx.grid_volume(grid)
+    for sd in (100.0, 140.0, 150.0):
+        want, wst = abi.build_octree(grid, heuristic=abi.HEURISTIC_STD_DEV, std_dev=sd)
+        got, gst = ctx.build_octree(gv, heuristic=abi.HEURISTIC_STD_DEV, std_dev=sd)
+        assert gst == wst, sd
+        assert np.array_equal(got, want), sd
+    gv.free()

@@ -298,11 +298,21 @@ __device__ __forceinline__ void block_sum_dd(double hi, double lo, double2* out)
     if (threadIdx.x == 0) *out = make_double2(hs[0], ls[0]);
 }
 
+// The grid's part of a node, in bricks along an axis, as a number of bits (its
+// power of two is less than twice the part).
+__host__ __device__ __forceinline__ uint32_t part_bits(uint64_t origin, uint32_t extent, uint32_t bricks) {
+    const uint64_t left = bricks - (origin >> 2);
+    const uint32_t n = left < extent >> 2 ? (uint32_t)left : extent >> 2;
+    return n <= 1 ? 0u : 32u - (uint32_t)__builtin_clz(n - 1);
+}
+
 // Part blockIdx.x of node blockIdx.y + first, a row of four texels a thread at a
-// time: rows part, part + parts, ... in blocks of 256.  The extent (8 or more)
-// is a power of two, so a row's place follows from its bits.  A block a node,
-// with divisions for every voxel, had left the upper levels on a few CUs: 4.7 ms
-// for a 128^3 grid, now 0.05.
+// time: rows part, part + parts, ... in blocks of 256.  The rows are those of the
+// grid's part of the node, each side rounded up to a power of two, so that a row's
+// place follows from its bits: never more than eight times the rows that there are,
+// while the whole node's would be side^3 / 4 however thin the grid is.  A block a
+// node, with divisions for every voxel, had left the upper levels on a few CUs: 4.7
+// ms for a 128^3 grid, now 0.05.
 __global__ __launch_bounds__(256) void k_stddev_big(GridDev g, const uint64_t* codes, uint64_t first, uint32_t level,
                                                     uint32_t extent, Cells stats, double2* out) {
     const uint64_t i = first + blockIdx.y;
@@ -313,13 +323,14 @@ __global__ __launch_bounds__(256) void k_stddev_big(GridDev g, const uint64_t* c
     if (ox < g.X && oy < g.Y && oz < g.Z) {
         double avg[4];
         sd_avg(stats.at(cx, cy, cz), avg);
-        const uint32_t b = 29u - __builtin_clz(extent);  // log2 of the extent in bricks
-        const uint64_t rows = (uint64_t)extent * extent * extent / 4;
+        const uint32_t bxs = part_bits(ox, extent, g.nbx), bys = part_bits(oy, extent, g.nby),
+                       bzs = part_bits(oz, extent, g.nbz);
+        const uint64_t rows = 16ull << (bxs + bys + bzs), mx = (1ull << bxs) - 1, my = (1ull << bys) - 1;
         for (uint64_t k = (uint64_t)blockIdx.x * 256 + threadIdx.x; k < rows; k += (uint64_t)gridDim.x * 256) {
             const uint32_t r = (uint32_t)k & 15u;
             const uint64_t brick = k >> 4;
-            const uint32_t m = (1u << b) - 1u;
-            const uint64_t bx = (ox >> 2) + (brick & m), by = (oy >> 2) + (brick >> b & m), bz = (oz >> 2) + (brick >> (2 * b));
+            const uint64_t bx = (ox >> 2) + (brick & mx), by = (oy >> 2) + (brick >> bxs & my),
+                           bz = (oz >> 2) + (brick >> (bxs + bys));
             if (bx >= g.nbx || by * 4 + (r & 3u) >= g.Y || bz * 4 + (r >> 2) >= g.Z) continue;
             const uint4 v = *reinterpret_cast<const uint4*>(g.bricks + ((bz * g.nby + by) * g.nbx + bx) * 64 + r * 4);
             const uint32_t w[4] = {v.x, v.y, v.z, v.w};
@@ -701,9 +712,10 @@ int xd_build_octree_device(xd_context* ctx, const xd_volume* grid, int heuristic
             XD_TRY(hipMemsetAsync(amb_n, 0, 4, s), "octree build: std-dev");
             if (from_pyr && extent >= 8) {
                 // parts of at least 4096 voxels, enough of them to fill the device
-                const uint64_t voxels = (uint64_t)extent * extent * extent;
+                const uint64_t bricks = 1ull << (part_bits(0, extent, g.nbx) + part_bits(0, extent, g.nby) +
+                                                 part_bits(0, extent, g.nbz));
                 const uint32_t parts =
-                    (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(voxels / 4096, (4096 + n - 1) / n));
+                    (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(bricks / 64, (4096 + n - 1) / n));
                 double2* part = nullptr;
                 XD_TRY(alloc((void**)&big, n * sizeof(double2)), "octree build: std-dev");
                 XD_TRY(alloc((void**)&part, n * parts * sizeof(double2)), "octree build: std-dev");
