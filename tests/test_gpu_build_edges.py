@@ -78,3 +78,17 @@ def test_std_dev_of_thin_grids(ctx, dims):
         assert gst == wst, sd
         assert np.array_equal(got, want), sd
     gv.free()
+
+
+def test_side_limit(ctx):
+    """Node codes hold 21 levels: a grid of 2^21 voxels a side is converted, a longer one refused."""
+    line = np.zeros((1, 1, (1 << 21) + 1, 4), np.uint8)
+    gv = ctx.grid_volume(line[:, :, :-1])
+    nodes, st = ctx.build_octree(gv)
+    assert st["side"] == 1 << 21 and len(nodes) == 1 + 8 * ((1 << 21) - 1)
+    gv.free()
+    gv = ctx.grid_volume(line)
+    with pytest.raises(abi.XdError) as err:
+        ctx.build_octree(gv)
+    assert err.value.status == abi.XD_ERR_FORMAT
+    gv.free()

@@ -170,6 +170,9 @@ __global__ void k_stats_merge(Cells child, Cells out) {
     out.s[i] = s;
 }
 
+// A node's code holds three bits for each level above it.
+constexpr uint32_t kMaxCodeLevels = 21;
+
 __device__ __forceinline__ void decode(uint64_t code, uint32_t level, uint32_t& x, uint32_t& y, uint32_t& z) {
     x = y = z = 0;
     for (uint32_t l = 0; l < level; ++l) {
@@ -610,6 +613,9 @@ int xd_build_octree_device(xd_context* ctx, const xd_volume* grid, int heuristic
     while (side < std::max({grid->dims[0], grid->dims[1], grid->dims[2]})) side <<= 1;
     uint32_t D = 0;
     while ((1ull << D) < side) ++D;
+    if (D > kMaxCodeLevels)
+        return fail(XD_ERR_FORMAT, "octree of %llu voxels a side is too large for the device build (limit 2^%u)",
+                    (unsigned long long)side, kMaxCodeLevels);
     const GridDev g{grid->d_bricks, (uint32_t)grid->dims[0], (uint32_t)grid->dims[1], (uint32_t)grid->dims[2],
                     grid->nb[0], grid->nb[1], grid->nb[2]};
 
