@@ -1,0 +1,37 @@
+"""Grids and trees whose kernels need more threads than one launch may have
+(2^32 along an axis): a plane of 2^32 voxels, and a level of 2^24 nodes."""
+import numpy as np
+import pytest
+
+from oracle import xo
+from xenodon_amd import abi
+
+pytestmark = [pytest.mark.gpu, pytest.mark.timeout(300)]
+
+SIDE = 1 << 16
+
+
+@pytest.fixture(scope="module")
+def plane():
+    """65536 x 65536 x 1 voxels, a few of them coloured, the last among them; 2^28 bricks."""
+    if abi.device_count() < 1:
+        pytest.fail("no HIP device visible: GPU tests need an MI355X")
+    grid = np.zeros((1, SIDE, SIDE, 4), np.uint8)
+    at = [(SIDE - 1, SIDE - 1), (SIDE - 1, SIDE - 2), (SIDE - 3, 5), (SIDE // 2, SIDE - 1)]  # y, x
+    for k, (y, x) in enumerate(at):
+        grid[0, y, x] = (200, 40 + 50 * k, 90, 255)
+    with abi.Context(0) as ctx:
+        yield ctx, grid, ctx.grid_volume(grid), at
+
+
+def test_bricks_of_a_plane_of_2_32_voxels(plane):
+    ctx, grid, vol, at = plane
+    ov = xo.OracleVolume(grid=grid)
+    for y, x in at:
+        eye = ((x + 0.5) / SIDE, (y + 0.5) / SIDE, -4.0 / SIDE)
+        cam = (0.0, 0.0, 1.0), (0.0, 1.0, 0.0), eye
+        args = (31, 31, [SIDE, SIDE, 1])
+        got, _ = ctx.render_image(vol, abi.DDA, abi.make_camera(*cam), abi.make_uniforms(*args, emission=3e4))
+        want = xo.render(abi.DDA, ov, xo.make_camera(*cam), xo.make_uniforms(*args, emission=3e4))["rgba"]
+        assert want[..., :3].any()
+        assert np.array_equal(got, want), (y, x)

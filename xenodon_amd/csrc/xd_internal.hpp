@@ -59,6 +59,10 @@ constexpr uint32_t kTableLevelMask = 0xFFu, kTableLowNode = 0x100u;
 constexpr uint32_t kRopeCellFirst = kTableLevel, kRopeCellLast = 12;
 constexpr uint32_t kRecWords = 12;  // words of an internal node's record (RenderParams::rec)
 
+// Blocks of 256 threads in one launch: the threads along a grid's axis are counted in
+// 32 bits.  More take several launches.
+constexpr uint64_t kMaxBlocks256 = 0xFFFFFFFFull / 256;
+
 // Everything one traversal launch needs; passed by value as the kernel
 // argument (kernarg segment), so a launch needs no device-side setup.
 struct RenderParams {

@@ -12,6 +12,8 @@
 // and walk neighbouring voxels/nodes (coherent gathers through L2).  The
 // hardware deals blocks to the 8 XCDs round-robin, and by default neighbouring
 // blocks stay on different XCDs (see block_pixel).
+#include <algorithm>
+
 #include "xd_trace.hpp"
 
 namespace xd {
@@ -121,9 +123,10 @@ hipError_t launch_traversal(int traversal, int tile_w, bool count_words, const R
 // read and written in 63 us, 4.7 TB/s.  One thread a brick, a launch a layer,
 // had taken 2.3 ms.
 __global__ __launch_bounds__(256) void k_bricks(const uint32_t* __restrict__ staging, uint32_t layers, uint64_t first,
-                                                uint64_t rows, uint32_t* __restrict__ bricks, uint8_t* __restrict__ occ,
-                                                uint32_t X, uint32_t Y, uint32_t nbx, uint32_t nby) {
-    const uint64_t g = (uint64_t)blockIdx.x * 256 + threadIdx.x;
+                                                uint64_t block0, uint64_t rows, uint32_t* __restrict__ bricks,
+                                                uint8_t* __restrict__ occ, uint32_t X, uint32_t Y, uint32_t nbx,
+                                                uint32_t nby) {
+    const uint64_t g = (block0 + blockIdx.x) * 256 + threadIdx.x;
     const bool live = g < rows;
     const uint32_t j = (uint32_t)(g >> 4), r = (uint32_t)g & 15u;
     uint4 v = make_uint4(0, 0, 0, 0);
@@ -178,8 +181,10 @@ hipError_t launch_macro_mask(const uint8_t* occ, const uint32_t nb[3], uint32_t 
 hipError_t launch_bricks(const uint32_t* staging, uint32_t layers, uint32_t bz, uint32_t* bricks, uint8_t* occ,
                          const uint32_t dims[3], const uint32_t nb[3], hipStream_t s) {
     const uint64_t per_layer = (uint64_t)nb[0] * nb[1], rows = per_layer * ((layers + kBrick - 1) / kBrick) * 16;
-    hipLaunchKernelGGL(k_bricks, dim3((uint32_t)((rows + 255) / 256)), dim3(256), 0, s, staging, layers, bz * per_layer,
-                       rows, bricks, occ, dims[0], dims[1], nb[0], nb[1]);
+    const uint64_t blocks = (rows + 255) / 256;
+    for (uint64_t b = 0; b < blocks; b += kMaxBlocks256)
+        hipLaunchKernelGGL(k_bricks, dim3((uint32_t)std::min(kMaxBlocks256, blocks - b)), dim3(256), 0, s, staging, layers,
+                           bz * per_layer, b, rows, bricks, occ, dims[0], dims[1], nb[0], nb[1]);
     return hipGetLastError();
 }
 
