@@ -35,3 +35,27 @@ def test_bricks_of_a_plane_of_2_32_voxels(plane):
         want = xo.render(abi.DDA, ov, xo.make_camera(*cam), xo.make_uniforms(*args, emission=3e4))["rgba"]
         assert want[..., :3].any()
         assert np.array_equal(got, want), (y, x)
+
+
+def test_statistics_of_2_28_bricks():
+    """4096 x 2048 x 2048 voxels, a few of them coloured: the tree down to each of these from the root, and every other
+    leaf empty."""
+    grid = np.zeros((2048, 2048, 4096, 4), np.uint8)
+    at = [(4095, 2047, 2047), (0, 0, 2047), (4094, 3, 1029), (2047, 2047, 0)]  # x, y, z
+    for k, (x, y, z) in enumerate(at):
+        grid[z, y, x] = (200, 40 + 50 * k, 90, 255)
+    with abi.Context(0) as ctx:
+        nodes, st = ctx.build_octree(ctx.grid_volume(grid))
+    assert st["side"] == 4096
+    leaf = nodes[:, 9] >= 1 << 31
+    seen = {0}
+    for x, y, z in at:
+        i = 0
+        for d in range(12):
+            assert not leaf[i] and nodes[i, 9] == d
+            i = int(nodes[i, (x >> (11 - d) & 1) << 2 | (y >> (11 - d) & 1) << 1 | (z >> (11 - d) & 1)])
+            seen.add(i)
+        assert nodes[i, 9] == 0x8000000C and nodes[i, 8] == grid[z, y, x].view(np.uint32)[0]
+    assert len(nodes) == 1 + 8 * sum(not leaf[i] for i in seen)
+    leaf[list(seen)] = False
+    assert not nodes[leaf, 8].any()

@@ -115,8 +115,8 @@ struct Cells {
 // Level of 4^3 cells, a cell's 16 rows in a quarter of a wave: a
 // lane takes its row's four texels with one load, and the quarter adds them up.
 // A thread a cell, with 64 loads, took 250 us for a 300x217x283 grid.
-__global__ __launch_bounds__(256) void k_stats_base(GridDev g, Cells out) {
-    const uint64_t t = (uint64_t)blockIdx.x * 256 + threadIdx.x, i = t >> 4;
+__global__ __launch_bounds__(256) void k_stats_base(GridDev g, uint64_t block0, Cells out) {
+    const uint64_t t = (block0 + blockIdx.x) * 256 + threadIdx.x, i = t >> 4;
     const uint32_t r = (uint32_t)t & 15u;
     const uint64_t cells = (uint64_t)out.nx * out.ny * out.nz;  // the bricks, in their order
     uint32_t n = 0, sum[4] = {0, 0, 0, 0}, mn = 0xFFFFFFFFu, mx = 0;
@@ -682,7 +682,9 @@ int xd_build_octree_device(xd_context* ctx, const xd_volume* grid, int heuristic
         const uint64_t n = (uint64_t)c.nx * c.ny * c.nz;
         XD_TRY(alloc((void**)&c.s, n * sizeof(CellStats)), "octree build: statistics");
         if (L == B)
-            hipLaunchKernelGGL(k_stats_base, dim3(blocks_for(n * 16)), dim3(256), 0, s, g, c);
+            for (uint64_t b = 0, count = (n * 16 + 255) / 256; b < count; b += kMaxBlocks256)
+                hipLaunchKernelGGL(k_stats_base, dim3((unsigned)std::min(kMaxBlocks256, count - b)), dim3(256), 0, s, g, b,
+                                   c);
         else
             hipLaunchKernelGGL(k_stats_merge, dim3(blocks_for(n)), dim3(256), 0, s, pyr[L + 1], c);
         XD_TRY(hipGetLastError(), "octree build: statistics");
