@@ -59,3 +59,19 @@ def test_statistics_of_2_28_bricks():
     assert len(nodes) == 1 + 8 * sum(not leaf[i] for i in seen)
     leaf[list(seen)] = False
     assert not nodes[leaf, 8].any()
+
+
+def test_standard_deviation_of_a_level_of_2_24_nodes():
+    """32768 x 16384 x 8 voxels: nodes of 16 voxels a side reach out of the grid and are split, 8 into each.  Of those
+    some hold two colours, far enough apart for either heuristic, so the two give one tree."""
+    grid = np.zeros((8, 16384, 32768, 4), np.uint8)
+    rng = np.random.default_rng(3)
+    for x, y in [(4095, 2047), (0, 0)] + [(rng.integers(4096), rng.integers(2048)) for _ in range(60)]:
+        grid[:, 8 * y:8 * y + 8, 8 * x:8 * x + 4] = rng.integers(100, 256, 4)
+    with abi.Context(0) as ctx:
+        vol = ctx.grid_volume(grid)
+        want, _ = ctx.build_octree(vol, heuristic=abi.HEURISTIC_CHAN_DIFF, chan_diff=20)
+        got, _ = ctx.build_octree(vol, heuristic=abi.HEURISTIC_STD_DEV, std_dev=5.0)
+    level = got[:, 9] & 0xFF
+    assert (level == 12).sum() >= 1 << 24 and (level == 13).any()
+    assert np.array_equal(got, want)

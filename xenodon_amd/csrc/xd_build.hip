@@ -730,12 +730,16 @@ int xd_build_octree_device(xd_context* ctx, const xd_volume* grid, int heuristic
                 for (uint64_t first = 0; first < n; first += 65535)  // the grid's second dimension
                     hipLaunchKernelGGL(k_stddev_big, dim3(parts, (unsigned)std::min<uint64_t>(65535, n - first)), dim3(256),
                                        0, s, g, cur.codes, first, L, extent, pyr[L], part);
-                hipLaunchKernelGGL(k_stddev_join, dim3((unsigned)n), dim3(256), 0, s, part, parts, big);
+                for (uint64_t first = 0; first < n; first += kMaxBlocks256)
+                    hipLaunchKernelGGL(k_stddev_join, dim3((unsigned)std::min(kMaxBlocks256, n - first)), dim3(256), 0, s,
+                                       part + first * parts, parts, big + first);
+                XD_TRY(hipGetLastError(), "octree build: std-dev");  // or the sums would be read unwritten
             }
         }
         hipLaunchKernelGGL(k_classify, dim3(blocks_for(n)), dim3(256), 0, s, g, cur.codes, n, L, extent,
                            from_pyr ? pyr[L] : Cells{}, sd ? 1u : 0u, (uint32_t)chan_diff, std_dev, big, amb,
                            amb_n, cur.colour, cur.internal);
+        XD_TRY(hipGetLastError(), "octree build: classify");
         if (sd) {
             // nodes too close to the limit to decide on the device: the
             // reference's sequential S, and the converter's own comparison
