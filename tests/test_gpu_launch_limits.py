@@ -37,6 +37,15 @@ def test_bricks_of_a_plane_of_2_32_voxels(plane):
         assert np.array_equal(got, want), (y, x)
 
 
+def test_a_level_too_large_to_scan_is_refused(plane):
+    """Every node of a plane is split down to the voxels: 2^31 nodes of 2 voxels a side, more than the scans count."""
+    ctx, _, vol, _ = plane
+    for tree in (abi.TREE_SPARSE, abi.TREE_DAG):
+        with pytest.raises(abi.XdError) as err:
+            ctx.build_octree(vol, tree=tree)
+        assert err.value.status == abi.XD_ERR_FORMAT
+
+
 def test_statistics_of_2_28_bricks():
     """4096 x 2048 x 2048 voxels, a few of them coloured: the tree down to each of these from the root, and every other
     leaf empty."""

@@ -577,6 +577,9 @@ __global__ void k_ropes(const uint64_t* codes, uint64_t count, uint32_t level, u
     for (int k = 0; k < 6; ++k) nodes[(uint64_t)fi * 10 + k] = r[k];
 }
 
+// Items of a scan or a sort, which count them in an int.
+constexpr uint64_t kMaxScan = 0x7FFFFFFFull;
+
 inline unsigned blocks_for(uint64_t n) { return (unsigned)((n + 255) / 256); }
 
 struct Level {
@@ -703,10 +706,6 @@ int xd_build_octree_device(xd_context* ctx, const xd_volume* grid, int heuristic
         Level& cur = lv[L];
         const uint64_t n = cur.count;
         total += n;
-        if (total > 0xFFFFFFFFull) {
-            cleanup();
-            return fail(XD_ERR_FORMAT, "octree exceeds 2^32 nodes");
-        }
         XD_TRY(alloc((void**)&cur.colour, n * 4), "octree build: lists");
         XD_TRY(alloc((void**)&cur.internal, n * 4), "octree build: lists");
         XD_TRY(alloc((void**)&cur.rank, n * 4), "octree build: lists");
@@ -784,6 +783,15 @@ int xd_build_octree_device(xd_context* ctx, const xd_volume* grid, int heuristic
         if (internals == 0) break;
         Level next;
         next.count = internals * 8;
+        if (total + next.count > 0xFFFFFFFFull) {
+            cleanup();
+            return fail(XD_ERR_FORMAT, "octree exceeds 2^32 nodes");
+        }
+        if (next.count > kMaxScan) {
+            cleanup();
+            return fail(XD_ERR_FORMAT, "octree level of %llu nodes is too large for the device build",
+                        (unsigned long long)next.count);
+        }
         XD_TRY(alloc((void**)&next.codes, next.count * 8), "octree build: lists");
         hipLaunchKernelGGL(k_children, dim3(blocks_for(n)), dim3(256), 0, s, cur.codes, n, cur.internal, cur.rank,
                            next.codes);
@@ -810,17 +818,17 @@ int xd_build_octree_device(xd_context* ctx, const xd_volume* grid, int heuristic
     unsigned long long unique_leaves = leaves;
     uint32_t* ins = nullptr;
     if (dag) {
+        if (total > kMaxScan) {
+            cleanup();
+            return fail(XD_ERR_FORMAT, "octree of %llu nodes is too large for the device DAG build",
+                        (unsigned long long)total);
+        }
         unsigned long long* d_unique = nullptr;
         XD_TRY(alloc((void**)&d_unique, 8), "octree build: dag");
         XD_TRY(hipMemsetAsync(d_unique, 0, 8, s), "octree build: dag");
         for (int L = (int)depth; L >= 0; --L) {
             Level& cur = lv[L];
             const uint64_t n = cur.count;
-            if (n > 0x7FFFFFFFull) {
-                cleanup();
-                return fail(XD_ERR_FORMAT, "octree level of %llu nodes is too large for the device DAG build",
-                            (unsigned long long)n);
-            }
             const uint32_t* cls_child = L < (int)depth ? lv[L + 1].cls : nullptr;
             uint64_t *k0 = nullptr, *k1 = nullptr;
             uint32_t *i0 = nullptr, *i1 = nullptr, *head = nullptr, *run = nullptr;
