@@ -583,7 +583,10 @@ int upload_tables(xd_batch* b, BatchClasses* need) {
     if ((rc = ensure_capacity(b, n, std::max<uint32_t>(T.total_tiles, 1)))) return rc;
     hipError_t e;
     hipStream_t s = b->ctx->stream;
-    if ((e = hipMemcpyAsync(b->d_views, T.views.data(), sizeof(BatchView) * n, hipMemcpyHostToDevice, s)) != hipSuccess ||
+    // the frames' device memory is the program's too: what it has queued on the null
+    // stream comes before the renders of these views, as it did before a hipMemcpy
+    if ((e = hipStreamSynchronize(nullptr)) != hipSuccess ||
+        (e = hipMemcpyAsync(b->d_views, T.views.data(), sizeof(BatchView) * n, hipMemcpyHostToDevice, s)) != hipSuccess ||
         (e = hipMemcpyAsync(b->d_qbeg, T.qbeg, sizeof(T.qbeg), hipMemcpyHostToDevice, s)) != hipSuccess ||
         (e = write_tiles(T, b->tuning.interleave, b->d_views, b->d_tiles, s)) != hipSuccess ||
         (e = hipStreamSynchronize(s)) != hipSuccess) {

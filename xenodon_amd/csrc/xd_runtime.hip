@@ -600,6 +600,8 @@ int xd_volume_from_svo(xd_context* ctx, const void* nodes, uint64_t node_count, 
     const uint32_t* w = static_cast<const uint32_t*>(nodes);
     hipError_t e = hipSetDevice(ctx->device);
     if (e != hipSuccess) return fail_hip(e, "hipSetDevice");
+    // as the copies of an upload on the null stream would wait for what the program has there
+    if ((e = hipStreamSynchronize(nullptr)) != hipSuccess) return fail_hip(e, "octree upload");
     auto* v = new xd_volume();
     v->ctx = ctx;
     v->kind = XD_VOLUME_SVO;
