@@ -236,7 +236,9 @@ class Context:
 
     def close(self):
         if self.h:
-            # xd_close frees the context's remaining volumes and frames
+            # xd_close frees the context's remaining volumes and frames.  The collector
+            # takes weak references to what goes with the context first, so a child looks
+            # at its context's handle as well.
             for c in list(self._children):
                 c.h = None
             lib().xd_close(self.h)
@@ -427,9 +429,9 @@ class Batch:
         return ms.value, rays.value
 
     def free(self):
-        if self.h:
+        if self.h and self.ctx.h:
             lib().xd_batch_free(self.h)
-            self.h = None
+        self.h = None
 
     def __del__(self):
         try:
@@ -510,9 +512,9 @@ class Server:
         return lib().xd_server_now_ms(self.h)
 
     def free(self):
-        if self.h:
+        if self.h and self.ctx.h:
             lib().xd_server_free(self.h)
-            self.h = None
+        self.h = None
 
     def __del__(self):
         try:
@@ -540,9 +542,9 @@ class Volume:
         return i
 
     def free(self):
-        if self.h:
+        if self.h and self.ctx.h:
             lib().xd_volume_free(self.h)
-            self.h = None
+        self.h = None
 
     def __del__(self):
         try:
@@ -569,9 +571,9 @@ class Frame:
         return p.value
 
     def free(self):
-        if self.h:
+        if self.h and self.ctx.h:
             lib().xd_frame_free(self.h)
-            self.h = None
+        self.h = None
 
     def __del__(self):
         try:
