@@ -66,3 +66,37 @@ def test_dda_runs_match_the_oracle(ctx, dims, scale):
         for v in views:
             v[4].free()
         gv.free()
+
+
+@pytest.mark.parametrize("scale", [1.0, 1.7])
+@pytest.mark.parametrize("dims", DIMS)
+def test_dda_runs_in_the_kernel_of_all_traversals(ctx, dims, scale):
+    """An octree view beside them takes the DDA views to that kernel, whose batches of steps are shorter.  The frames
+    hold black before each launch."""
+    md = [max(1, int(round(d * scale))) for d in dims]
+    grid = _lone_voxels(dims, 1)
+    ov, gv = xo.OracleVolume(grid=grid), ctx.grid_volume(grid)
+    nodes, st = abi.build_octree(H.blocky_grid(16, 4, seed=5))
+    sv = ctx.svo_volume(nodes, st["side"])
+    away = abi.make_camera(*H.look_at((0.5, 0.5, 3.0), (0.5, 0.5, 9.0)))
+    views, refs = [], []
+    for f, up, eye in CAMERAS:
+        refs.append(xo.render(abi.DDA, ov, xo.make_camera(f, up, eye), xo.make_uniforms(61, 43, md, emission=0.8))["rgba"])
+        views.append((gv, abi.DDA, abi.make_camera(f, up, eye), abi.make_uniforms(61, 43, md, emission=0.8),
+                      ctx.frame(61, 43)))
+    tree = (sv, abi.ESVO, away, abi.make_uniforms(9, 9, [st["side"]] * 3), ctx.frame(9, 9))
+    b = ctx.batch()
+    b.set_tuning([8] * 5, class_kernels=0)
+    for launch in (lambda: (b.set_views(views + [tree]), b.render()),
+                   lambda: abi.render_static(ctx, views + [tree], {"tile_w": [8] * 5, "class_kernels": 0})):
+        for v in views:
+            ctx.render(gv, abi.DDA, away, v[3], v[4])
+            assert not v[4].download()[..., :3].any()
+        launch()
+        for v, ref in zip(views, refs):
+            assert np.array_equal(v[4].download(), ref), (dims, scale)
+    b.free()
+    for v in views + [tree]:
+        v[4].free()
+    gv.free()
+    sv.free()

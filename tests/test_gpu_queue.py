@@ -1,6 +1,8 @@
 """The batched forms' tile queues: launches from one wave tile up to more tiles
 than resident waves, growing and shrinking on one batch object (whose captured
 launch is reused), give the plain render's frames, bit for bit."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -78,3 +80,34 @@ def test_every_tile_is_dealt(env, order, tile_w, rpl):
         v[4].free()
     b.free()
     vol.free()
+
+
+@pytest.mark.parametrize("travs", [[abi.DDA], [abi.SVO_DF], TRAVERSALS])
+@pytest.mark.parametrize("class_kernels", [0, 1])
+def test_queue_sizes_on_frames_that_hold_something_else(env, travs, class_kernels):
+    """Each launch alone fills its frames: before it they hold bytes that no frame has (a pixel's last is 255)."""
+    ctx, grid, svo = env
+    hip = abi.lib()  # finds the HIP runtime's functions as well
+    hip.hipMemset.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_size_t]
+    b = ctx.batch()
+    b.set_tuning([8] * 5, class_kernels=class_kernels)
+    for n, W, Hh in SHAPES:
+        views = []
+        for k, (f, up, eye) in enumerate(H.orbit_cameras(n, 1.6, seed=n)):
+            t = travs[k % len(travs)]
+            vol, md = grid if t == abi.DDA else svo
+            views.append((vol, t, abi.make_camera(f, up, eye), abi.make_uniforms(W, Hh, md, emission=1.5),
+                          ctx.frame(W, Hh)))
+        refs = [ctx.render_image(*v[:4])[0] for v in views]
+        b.set_views(views)
+        for launch in (b.render, b.render,
+                       lambda: abi.render_static(ctx, views, {"tile_w": [8] * 5, "class_kernels": class_kernels})):
+            for v in views:
+                assert hip.hipMemset(v[4].device_ptr(), 0x55, W * Hh * 4) == 0
+                assert (v[4].download() == 0x55).all()
+            launch()
+            for v, ref in zip(views, refs):
+                assert np.array_equal(v[4].download(), ref), (n, W, Hh)
+        for v in views:
+            v[4].free()
+    b.free()

@@ -188,3 +188,48 @@ def test_ropes_into_the_near_corner_of_their_target(ctx, to, depth):
         changed += int((want != _pair(ctx, plain, side, abi.SVO_ROPE, cam, 41, 29)[1]).any())
         assert np.array_equal(got, want), int((got != want).any(-1).sum())
     assert changed  # or the ropes would not matter to these views
+
+
+@pytest.mark.parametrize("depth", [1, 2, 7, 8, 9, 10, 12, 14, 22])
+def test_naive_chain_trees(ctx, depth):
+    nodes = _tree(depth, abi.SVO_NAIVE, seed=depth)
+    for name, cam in CAMERAS.items():
+        got, want = _pair(ctx, nodes, 1 << depth, abi.SVO_NAIVE, cam())
+        assert np.array_equal(got, want), name
+
+
+@pytest.mark.parametrize("tree", [abi.TREE_SPARSE, abi.TREE_ROPE, abi.TREE_DAG])
+def test_naive_built_trees(ctx, tree):
+    nodes, st = abi.build_octree(_grid(), tree=tree)
+    for name, cam in CAMERAS.items():
+        got, want = _pair(ctx, nodes, st["side"], abi.SVO_NAIVE, cam())
+        assert np.array_equal(got, want), name
+
+
+@pytest.mark.parametrize("t, tree", [(t, abi.TREE_ROPE) for t in (abi.SVO_NAIVE, abi.ESVO, abi.SVO_DF, abi.SVO_ROPE)] +
+                         [(t, abi.TREE_DAG) for t in (abi.SVO_NAIVE, abi.ESVO, abi.SVO_DF)])
+def test_wide_tags_below_the_start_table(ctx, t, tree):
+    """31-bit indices without an empty tag, in trees of 10 levels: leaves and records below the table's 8."""
+    nodes, side, used = _corner_tree(10)
+    if tree == abi.TREE_DAG:
+        block = np.kron(_grid(), np.ones((2, 2, 2, 1), np.uint8))
+        grid = np.zeros((96, 96, 513, 4), np.uint8)
+        grid[:, :, 1:97] = block
+        nodes, st = abi.build_octree(grid, tree=tree)
+        side = st["side"]
+    vols = []
+    for layout in (RAW, 2):
+        ctx.set_option("octree_layout", layout)
+        try:
+            vols.append(ctx.svo_volume(nodes, side))
+        finally:
+            ctx.set_option("octree_layout", 0)
+    mid = 0.5 * used
+    near = [_camera((-0.8 * used, 1.4 * used, -1.1 * used), np.array([mid] * 3) - np.array((-0.8, 1.4, -1.1)) * used),
+            _camera((0.4 * used, 0.45 * used, 0.7 * used), (1.0, -0.7, -0.4))]
+    for cam in near + [make() for make in CAMERAS.values()]:
+        uni = abi.make_uniforms(61, 47, [side] * 3, emission=1.5)
+        want, got = (ctx.render_image(v, t, cam, uni)[0] for v in vols)
+        assert np.array_equal(got, want)
+    for v in vols:
+        v.free()
