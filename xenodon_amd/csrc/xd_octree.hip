@@ -34,7 +34,7 @@
 #include <vector>
 
 #include "xd_runtime.hpp"
-#include "xd_svo_fast.hpp"
+#include "xd_table.hpp"
 
 namespace xd {
 namespace {
@@ -313,32 +313,16 @@ __global__ __launch_bounds__(kOctBlock) void k_oct_emit(const uint2* __restrict_
     }
 }
 
-// One cell of the start table a thread: the walk of build_start_table.
+// One cell of the start table a thread.
 // stop: null, or a word that says, when set, that the child words are no tree's.
 __global__ __launch_bounds__(256) void k_start_table(const uint32_t* __restrict__ cw, uint32_t root_tag,
                                                      uint32_t index_mask, uint32_t shift,
                                                      const uint4* __restrict__ rec, const uint32_t* stop,
                                                      uint2* __restrict__ table) {
     if (stop && *stop) return;
-    uint32_t cell = blockIdx.x * 256 + threadIdx.x;
-    const uint32_t levels = kTableLevel - shift;
-    uint3 p = table_place(cell);
-    if (shift) {  // the cells below 2^levels of each axis
-        const uint32_t m = (1u << levels) - 1u, sh = 23u - levels;
-        if (cell >> (3 * levels)) return;
-        p = make_uint3((cell & m) << sh, (cell >> levels & m) << sh, (cell >> (2 * levels) & m) << sh);
-        cell = table_cell(p.x >> shift, p.y >> shift, p.z >> shift);
-    }
-    uint32_t word = root_tag, level = 0;
-    while (!(word & kTagLeaf) && level < levels) {
-        const uint32_t s = 22u - level;
-        const uint32_t k = (p.x >> s & 1u) << 2 | (p.y >> s & 1u) << 1 | (p.z >> s & 1u);
-        word = cw[(uint64_t)(word & index_mask) * 8 + k];
-        ++level;
-    }
-    if (!(word & kTagLeaf) && rec && (rec[(uint64_t)(word & index_mask) * (kRecWords / 4)].y & 0xFFu) == 0)
-        level |= kTableLowNode;
-    table[cell] = make_uint2(word, level);
+    uint32_t at;
+    uint2 entry;
+    if (table_entry(cw, root_tag, index_mask, shift, rec, blockIdx.x * 256 + threadIdx.x, &at, &entry)) table[at] = entry;
 }
 
 }  // namespace

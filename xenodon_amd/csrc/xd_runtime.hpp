@@ -55,7 +55,7 @@ struct xd_volume {
     uint32_t* d_nodes = nullptr;
     uint32_t* d_cw = nullptr;
     uint32_t* d_meta = nullptr;  // colours of all nodes, then their is_leaf_depth words
-    uint2* d_table = nullptr;  // start table of the tagged layout (see build_start_table)
+    uint2* d_table = nullptr;  // start table of the tagged layout (see launch_start_table)
     uint32_t rope_depth = 0;   // ropes carry their targets' depth fields (see pack_rope_depths)
     uint32_t index_mask = 0;   // index bits of the tagged child words
     uint32_t empty_tag = 0;    // kTagEmpty, or 0 for wide tags
@@ -129,11 +129,11 @@ bool octree_depths_exact(const uint32_t* w, uint64_t n, bool tree);
 // for any point of cell (x, y, z), or of the leaf that ends the walk above it;
 // that node's level}.  The root's word is 0 | root_tag.  The walk follows
 // child words for at most L levels, so any tree, cyclic ones included, gives
-// a table.
+// a table.  The plain statement of what the device's table holds, for checks.
 void build_start_table(const uint32_t* child_w, uint32_t root_tag, uint32_t index_mask, uint2* table);
 // The device's table, built there from the device form of child_w: the same
-// entries in the order of table_cell, with kTableLowNode from rec (or null).  stop:
-// null, or a device word that, if set, keeps the table unwritten.
+// entries in the order of table_cell (table_entry), with kTableLowNode from rec (or
+// null).  stop: null, or a device word that, if set, keeps the table unwritten.
 hipError_t launch_start_table(const uint32_t* cw, uint32_t root_tag, uint32_t index_mask, uint32_t shift, const uint4* rec,
                               const uint32_t* stop, uint2* table, hipStream_t s);
 // Derives v's tagged layout and start table on the device from n .svo nodes in

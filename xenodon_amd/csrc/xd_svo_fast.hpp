@@ -19,6 +19,7 @@
 #pragma once
 
 #include "xd_svo_ref.hpp"
+#include "xd_table.hpp"
 
 namespace xd {
 
@@ -113,21 +114,6 @@ __device__ __forceinline__ uint32_t clamp3(uint32_t x, uint32_t lo, uint32_t hi)
     uint32_t r;
     asm("v_med3_u32 %0, %1, %2, %3" : "=v"(r) : "v"(x), "v"(lo), "v"(hi));
     return r;
-}
-
-// Index in the start table of the cell at position bits (x, y, z): 4x4x4 cells
-// together, 512 B, as the rays of a tile walk neighbouring cells along any axis.
-__device__ __forceinline__ uint32_t table_cell(uint32_t x, uint32_t y, uint32_t z) {
-    constexpr uint32_t sh = 23u - kTableLevel, b = kTableLevel - 2;
-    return ((z >> (sh + 2)) << (2 * b) | (y >> (sh + 2)) << b | (x >> (sh + 2))) << 6 | (z >> sh & 3u) << 4 |
-           (y >> sh & 3u) << 2 | (x >> sh & 3u);
-}
-// Its inverse: the position bits of a cell's lower corner.
-__device__ __forceinline__ uint3 table_place(uint32_t cell) {
-    constexpr uint32_t sh = 23u - kTableLevel, b = kTableLevel - 2, m = (1u << b) - 1u;
-    return make_uint3((cell >> 6 & m) << (sh + 2) | (cell & 3u) << sh,
-                      (cell >> (b + 6) & m) << (sh + 2) | (cell >> 2 & 3u) << sh,
-                      (cell >> (2 * b + 6) & m) << (sh + 2) | (cell >> 4 & 3u) << sh);
 }
 
 // The index in s's table.  A branch that all lanes take alike: three shifts by 0 in
