@@ -127,11 +127,16 @@ void fill_params(RenderParams& p, const xd_volume* vol, int traversal, const xd_
         // the start table, and esvo / svo-df run at full occupancy with their
         // stacks alone in LDS (3 % faster than with the top levels beside them)
         // By the table on trees deeper than it (1080p frames of 9 levels 2 to 70 %
-        // faster, of 10 levels 0 to 55) and, where a launch waits for its loads more
-        // than it issues, on those as deep (eight frames each of 256^3 volumes: ct
-        // 1.98 -> 1.32 ms at 199x143, 1.79 -> 1.36 at 640x360, but 4.11 -> 4.44 at
-        // 1920x1080).  The ropes of a shallower tree stay in the caches better than
-        // the table's cells do: 0.36 -> 0.41 on 64^3, 0.64 -> 0.72 on 128^3.
+        // faster, of 10 levels 0 to 55) and, in frames below 2^20 pixels, on those as
+        // deep.  The line is the frame's, not the launch's, as measured: many small
+        // views in one launch gain about as one does, large ones lose (256^3
+        // volumes, by the ropes -> by the table: eight plain frames of 199x143 ct 2.35 ->
+        // 1.59 ms, 640x360 2.03 -> 1.52, 1280x720 2.61 -> 2.44, 1920x1080 4.03 -> 4.12; in
+        // one launch 40 of 199x143 1.40 -> 1.21, 40 of 640x360 2.29 -> 2.15, 16 of 1280x720
+        // 3.03 -> 3.05, 8 of 1920x1080 3.23 -> 3.37; shells and log-normal volumes are
+        // faster by the table at every size, 3 to 48 %).  The ropes of a shallower tree
+        // stay in the caches better than the table's cells do: 0.36 -> 0.41 on 64^3, 0.64
+        // -> 0.72 on 128^3.
         const uint64_t pixels = (uint64_t)u->output_region.extent[0] * u->output_region.extent[1];
         p.rope_cells = vol->rope_cells && (vol->max_depth > kTableLevel || pixels < (1u << 20)) ? 1u : 0u;
         p.top_nodes = !vol->d_cw || traversal != XD_SVO_ROPE || p.rope_cells ? 0u : vol->top[3];
